@@ -1,32 +1,53 @@
-// Chunked (WY-form) gated-delta prefill, fp32, gfx950.
+// Chunked (WY-form) gated-delta prefill, gfx950.
 //
 // The token recurrence of Q/src/reference.rs:230-297 / 377-415,
 //   S_t = a_t (I - b_t k_t k_t^T) S_{t-1} + b_t k_t v_t^T,   o_t = S_t^T q_t
 // (k, q L2-normalised, q also scaled by 1/sqrt(key_dim), a_t = exp(log_decay_t),
 // b_t = beta_t), is evaluated chunk by chunk. Within a chunk of C tokens, with
-// G_t = sum_{s<=t} log_decay_s (relative to the chunk start) and
-// g_t = exp(G_t):
+// G_t = sum_{s<=t} log_decay_s (relative to the chunk start) and g_t = exp(G_t):
 //   S_t = g_t S_0 + sum_{r<=t} exp(G_t - G_r) k_r d_r^T
-//   d_s = b_s (v_s - g_s S_0^T k_s - sum_{r<s} exp(G_s - G_r) (k_s.k_r) d_r)
-// i.e. (I + diag(b) M) D = diag(b) V - diag(b g) K S_0 with M the strictly
-// lower, decay-weighted K K^T, so D = T (diag(b) V - diag(b g) K S_0),
-// T = (I + diag(b) M)^{-1} (unit lower triangular). Then
+//   d_s = b_s (v_s - g_s S_0^T k_s - sum_{r<s} exp(G_s - G_r) (k_s.k_r) d_r).
+// With L the strictly lower b_s (k_s.k_r) and T0 = (I + L)^{-1} (no decay: the
+// decayed inverse is diag(g) T0 diag(1/g)), this is
+//   D   = U - diag(g) W S_0,   W = T0 diag(b) K,
+//                              U[s] = sum_{r<=s} exp(G_s - G_r) T0[s][r] b_r v_r
 //   O   = diag(g) Q S_0 + A D,       A[t][r] = exp(G_t - G_r) (q_t.k_r), r <= t
 //   S_C = g_C S_0 + sum_r exp(G_C - G_r) k_r d_r^T.
-// Every decay factor is exp of a non-positive difference (<= 1), so nothing
-// overflows however strong the decay.
+// Every decay factor is exp of a non-positive difference for decays <= 1, so
+// nothing overflows however strong the decay. Only D and S_C depend on the
+// chunks before, so all of W, U, A and the scaled rows of Q and K are made for
+// every chunk in parallel (pass 1) and the sequential pass 2 is two small
+// products deep per chunk.
 //
-// Pass 1 (ctox_gdn_chunk_prep_gfx950, one workgroup per (head, chunk), all
-// chunks in parallel): norms, G, M and A from the lower 16 x 16 tiles of
-// K K^T and Q K^T on v_mfma_f32_16x16x4_f32, T by
-// blocks: the four 16 x 16 diagonal blocks by forward substitution (a wave
-// each), the blocks below them on MFMA one block row at a time.
-// Pass 2 (ctox_gdn_chunk_scan_gfx950, one workgroup per (head, 16 value
-// columns), chunks in order): the 128 x 16 state slice stays in LDS across
-// chunks; the five small products per chunk run on v_mfma_f32_16x16x4_f32.
-// Value columns are independent in the recurrence, so slices need no
-// exchange. Padded tokens of a partial last chunk have k = q = v = 0,
+// Pass 1 (ctox_gdn_chunk_prep_gfx950, one workgroup per (head, chunk)): fp32
+// MFMA throughout; T0 by blocks: the four 16 x 16 diagonal blocks by forward
+// substitution (a wave each), the blocks below them on MFMA one block row at a
+// time. Its matrices leave as MFMA operands, see below.
+// Pass 2 (ctox_gdn_chunk_scan{1,2}_gfx950, one workgroup per (head, 16 or 32
+// value columns), chunks in order). Value columns are independent, so slices
+// need no exchange. Padded tokens of a partial chunk have k = q = v = 0,
 // beta = 0 and log_decay = 0: identity steps.
+//
+// Pass 2's products run on v_mfma_f32_16x16x32_f16 with every operand split
+// into an f16 high and low part (three MFMAs per product: hi hi + hi lo +
+// lo hi, fp32 accumulation): 16 times the fp32 MFMA rate for 22 significant
+// bits, at or under the fp32 products' own rounding (measured below). The
+// split is kept inside f16's range by powers of two that cost nothing: the
+// operands of pass 1 are scaled by 2^14 over their row's norm (which a factor
+// on the product's rows undoes), the state by 2^15 over each column's largest
+// magnitude per 32 keys, D by 2^15 over a bound of its column's (its operand
+// may be up to 2^10 below the bound before a bit is lost). fp32 inputs of any
+// magnitude therefore keep their precision.
+//
+// Pass 2 is a latency chain: per chunk the state operand, W S_0, D, its
+// exchange, K^T D. Four waves hold the state (fp32, in registers: wave w rows
+// 32 w .. 32 w + 31) and walk that chain; four more compute the outputs beside
+// them from the same two exchanges. The contraction index order of an operand
+// is free as long as both sides agree, and it is chosen so that a lane's MFMA
+// results are the very elements of its next operand: no transposes. Nothing
+// but the 8 KB state and 4 KB D operands passes through LDS; pass 1's operands
+// are read from memory in fragment order, one chunk ahead, straight to
+// registers.
 
 #include <hip/hip_runtime.h>
 
@@ -35,429 +56,659 @@
 
 #define GC 64        // max chunk length
 #define GKD 128      // max key_dim of the chunked path
-#define GVS 16       // value columns per pass-2 workgroup
-#define TPAD 65      // LDS row stride of T / A / M
+#define TPAD 65      // LDS row stride of L / T
+#define SPAD 132     // LDS row stride of K / Q rows
 
 typedef float gv4f __attribute__((ext_vector_type(4)));
+typedef _Float16 gh2 __attribute__((ext_vector_type(2)));
+typedef _Float16 gh8 __attribute__((ext_vector_type(8)));
+
+// Scratch of one (head, chunk), byte offsets. A fragment is one MFMA operand
+// of 16 rows x 32 contraction elements, [lane][8 halves]: lane (m = lane % 16,
+// g = lane / 16) holds row m's elements 4 g .. 4 g + 3 and 16 + 4 g .. + 3 of
+// the 32 (the order in which two 16 x 16 results hold them).
+#define GF_W 0                  // [token strip 4][key step 4][hi, lo][64 lanes][16 B]
+#define GF_K 32768              // K^T: [key tile 8][token step 2][hi, lo]
+#define GF_Q 65536              // as GF_W
+#define GF_A 98304              // [token strip 4][token step 2][hi, lo]
+#define GF_U 114688             // fp32 [value tile 8][token strip 4][64 lanes][4 rows]
+#define GF_AUX 147456           // floats: fw[64], fq[64], fa[64], mu[128], gC, fK, wn
+static_assert(GF_AUX + (3 * 64 + 128 + 3) * 4 <= CTOX_GDN_CHUNK_BYTES, "chunk scratch");
 
 __device__ __forceinline__ gv4f mfma4(float a, float b, gv4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-
-#define SPAD 132  // LDS row stride (floats) of pass-2 K / Q tiles and of S^T
-#define TSPAD 68  // LDS row stride of pass-2 T / A / Y^T / (b v)^T
-
-// 16 x 16 tile of A[16 x K] * B[K x 16] with both operands stored k-contiguous
-// (A row-major [m][k], B as B^T [n][k]): lane (m = l % 16, kq = l / 16)
-// covers k = kq * (K / 4) + u for MFMA u, so each lane reads a contiguous
-// run of K / 4 floats of both operands.
-template <int K, int LDA, int LDB>
-__device__ __forceinline__ gv4f tile_kk(const float *a, const float *bt, gv4f acc, uint32_t lane) {
-    const uint32_t m = lane & 15, kq = lane >> 4;
-    const float *ap = a + m * LDA + kq * (K / 4);
-    const float *bp = bt + m * LDB + kq * (K / 4);
-    // Four independent accumulation chains, summed at the end.
-    gv4f c1 = {0.0f, 0.0f, 0.0f, 0.0f}, c2 = c1, c3 = c1;
-#pragma unroll
-    for (int u = 0; u < K / 4; u += 4) {
-        const float4 av = *(const float4 *)(ap + u), bv = *(const float4 *)(bp + u);
-        acc = mfma4(av.x, bv.x, acc);
-        c1 = mfma4(av.y, bv.y, c1);
-        c2 = mfma4(av.z, bv.z, c2);
-        c3 = mfma4(av.w, bv.w, c3);
-    }
-    return (acc + c1) + (c2 + c3);
+__device__ __forceinline__ gv4f mfma_h(uint4 a, uint4 b, gv4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gh8, a), __builtin_bit_cast(gh8, b), c, 0, 0, 0);
+}
+// (hi + lo) x (hi + lo) without the lo lo term.
+__device__ __forceinline__ gv4f mfma_split(const uint4 (&a)[2], const uint4 (&b)[2], gv4f c) {
+    c = mfma_h(a[0], b[1], c);
+    c = mfma_h(a[1], b[0], c);
+    return mfma_h(a[0], b[0], c);
 }
 
-// Scratch per (head, chunk): T[64][64], A[64][64], then per token g = exp(G),
-// exp(G_C - G), kinv and kinv's counterpart for q times 1/sqrt(key_dim) g.
-__host__ __device__ constexpr uint32_t ctox_gdn_chunk_floats() { return 2 * GC * GC + 4 * GC; }
+// f16 high and low parts of two values. The values are rounded to fp32 first:
+// a product folded into one use's conversion and not into the other's gives
+// two different high parts next to a rounding boundary.
+__device__ __forceinline__ void split2(float x, float y, uint32_t &hi, uint32_t &lo) {
+    asm("" : "+v"(x), "+v"(y));
+    const gh2 h = {(_Float16)x, (_Float16)y};
+    const gh2 l = {(_Float16)(x - (float)h[0]), (_Float16)(y - (float)h[1])};
+    hi = __builtin_bit_cast(uint32_t, h);
+    lo = __builtin_bit_cast(uint32_t, l);
+}
+// A lane's fragment from two runs of four values.
+__device__ __forceinline__ void split8(gv4f a, gv4f b, uint4 (&f)[2]) {
+    split2(a[0], a[1], f[0].x, f[1].x);
+    split2(a[2], a[3], f[0].y, f[1].y);
+    split2(b[0], b[1], f[0].z, f[1].z);
+    split2(b[2], b[3], f[0].w, f[1].w);
+}
+// e with x < 2^e, kept where 2^(15 - e) and 2^(e - 15) are normal numbers
+// (a non-finite x takes the largest).
+__device__ __forceinline__ int exponent_of(float x) {
+    const int e = (int)((__float_as_uint(x) >> 23) & 255u) - 126;
+    return min(128, max(-110, e));
+}
+__device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
-extern "C" __global__ __launch_bounds__(256) void ctox_gdn_chunk_prep_gfx950(GdnArgs a) {
-    __shared__ __align__(16) float kh[GC * SPAD];
-    __shared__ __align__(16) float qh[GC * SPAD];  // q^ rows, then M (after the dot-product tiles)
-    __shared__ float G[GC], bt[GC], kinv_s[GC], qinv_s[GC];
-    float *mm = qh;
-    const uint32_t tid = threadIdx.x;
-    const uint32_t nch = (a.tokens + a.chunk - 1) / a.chunk;
-    const uint32_t h = blockIdx.x / nch, c = blockIdx.x % nch;
-    const uint32_t t0 = c * a.chunk;
+// Sum / max over the four lane groups (lanes l, l ^ 16, l ^ 32).
+__device__ __forceinline__ float groups_sum(float v) {
+    v += __shfl_xor(v, 16);
+    return v + __shfl_xor(v, 32);
+}
+__device__ __forceinline__ float groups_max(float v) {
+    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float((uint32_t)a[0]), __uint_as_float((uint32_t)a[1]));
+    a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float((uint32_t)a[0]), __uint_as_float((uint32_t)a[1]));
+}
+
+// 16 x 16 tile of (rows of A) x (rows of B)^T over key_dim on fp32 MFMA: both
+// operands in fragment order, a lane's 32 values of its row in 8 runs of four
+// (run u at columns 16 u + 4 g). a: LDS row of lane m16, offset by 4 g.
+__device__ __forceinline__ gv4f tile_rows(const float *a, const gv4f (&b)[8]) {
+    // Four independent accumulation chains, summed at the end.
+    gv4f c0 = {0.0f, 0.0f, 0.0f, 0.0f}, c1 = c0, c2 = c0, c3 = c0;
+#pragma unroll
+    for (int u = 0; u < 8; u++) {
+        const gv4f av = *(const gv4f *)(a + 16 * u);
+        c0 = mfma4(av[0], b[u][0], c0);
+        c1 = mfma4(av[1], b[u][1], c1);
+        c2 = mfma4(av[2], b[u][2], c2);
+        c3 = mfma4(av[3], b[u][3], c3);
+    }
+    return (c0 + c1) + (c2 + c3);
+}
+
+// Workgroup b runs on XCD b % 8. All workgroups of a head are placed on one
+// XCD, so that they share the head's operands in that XCD's L2: XCD x takes
+// heads x, x + 8, ..., `per` workgroups each (grid 8 * ceil(heads / 8) * per).
+__device__ __forceinline__ void head_of_block(uint32_t block, uint32_t per, uint32_t &h, uint32_t &i) {
+    const uint32_t q = block >> 3;
+    h = (block & 7) + 8 * (q / per);
+    i = q % per;
+}
+
+// Four values at columns col .. col + 3 of a row of `width` values (zeros past
+// it, or all when !ok). VEC: width a multiple of 4 and the row 16-byte aligned;
+// a compile-time choice, since a load behind a branch is waited for at its end.
+template <bool VEC>
+__device__ __forceinline__ gv4f load4(const float *row, uint32_t col, uint32_t width, bool ok) {
+    gv4f r;
+    if (VEC) {
+        ok = ok && col < width;
+        r = *(const gv4f *)(row + (ok ? col : 0));
+#pragma unroll
+        for (int x = 0; x < 4; x++) r[x] = ok ? r[x] : 0.0f;
+    } else {
+#pragma unroll
+        for (int x = 0; x < 4; x++) r[x] = ok && col + x < width ? row[col + x] : 0.0f;
+    }
+    return r;
+}
+
+// Bound by latency: one workgroup is a chain of about a dozen LDS exchanges
+// around 320 fp32 MFMAs per wave. K, Q and V are requested up front, Q stays in
+// registers and V waits in them for K's LDS rows, T0 replaces L in place, so
+// 52 KB of LDS let three workgroups share a CU.
+template <bool VEC>
+__device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
+    __shared__ __align__(16) float kh[GC * SPAD];  // raw K rows, then V rows
+    __shared__ float tt[GC * TPAD];                // L, T0, W's and then U's left operand
+    __shared__ float G[GC], bt[GC], kinv_s[GC], ekf[GC];
+    __shared__ float wsq[4][GC];
+    const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t m16 = lane & 15, g = lane >> 4;
+    uint32_t h, ci;
+    head_of_block(blockIdx.x, a.chunks, h, ci);
+    if (h >= a.heads) return;
+    const uint32_t t0 = (a.chunk0 + ci) * a.chunk;
     const uint32_t n = min(a.chunk, a.tokens - t0);
-    const uint32_t dk = a.key_dim;
+    const uint32_t dk = a.key_dim, dv = a.value_dim;
+    char *base = (char *)a.norms + ((size_t)h * a.chunks + ci) * CTOX_GDN_CHUNK_BYTES;
+    float *aux = (float *)(base + GF_AUX);
     const float qscale = 1.0f / sqrtf((float)dk);
+    const uint32_t own = 16 * w + m16;  // this lane's token of strip w
 
-    // Raw k, q rows into LDS (zeros beyond n rows and key_dim columns), four
-    // threads per row accumulating the squares. The tiles below use the raw
-    // rows and scale their products by the inverse norms.
+    const size_t th = (size_t)(t0 + min(lane, n - 1)) * a.heads + h;
+    const float ld_raw = a.log_decay[th], bt_raw = a.beta[th];
+    gv4f kr[8], qr[8], vr[8];
     {
-        const uint32_t s = tid >> 2, p = tid & 3;
-        float sk = 0.0f, sq = 0.0f;
-        if (s < n) {
-            const size_t qk = (size_t)(t0 + s) * a.qk_stride + (size_t)(h / a.rep) * dk;
-            const float *kr = a.k + qk;
-            const float *qr = a.q + qk;
-            for (uint32_t i = p; i < dk; i += 4) {
-                const float kv = kr[i], qv = qr[i];
-                kh[s * SPAD + i] = kv;
-                qh[s * SPAD + i] = qv;
-                sk += kv * kv;
-                sq += qv * qv;
-            }
-        }
-        for (uint32_t i = (s < n ? dk : 0) + p; i < GKD; i += 4) {
-            kh[s * SPAD + i] = 0.0f;
-            qh[s * SPAD + i] = 0.0f;
-        }
-        sk += __shfl_xor(sk, 1);
-        sk += __shfl_xor(sk, 2);
-        sq += __shfl_xor(sq, 1);
-        sq += __shfl_xor(sq, 2);
-        if (p == 0) {
-            kinv_s[s] = s < n ? 1.0f / sqrtf(sk + 1e-6f) : 0.0f;
-            qinv_s[s] = s < n ? 1.0f / sqrtf(sq + 1e-6f) : 0.0f;
+        const size_t row = (size_t)(t0 + min(own, n - 1)) * a.qk_stride + (size_t)(h / a.rep) * dk;
+#pragma unroll
+        for (int u = 0; u < 8; u++) kr[u] = load4<VEC>(a.k + row, 16 * u + 4 * g, dk, own < n);
+#pragma unroll
+        for (int u = 0; u < 8; u++) qr[u] = load4<VEC>(a.q + row, 16 * u + 4 * g, dk, own < n);
+#pragma unroll
+        for (int u = 0; u < 8; u++) {
+            const uint32_t s = (tid >> 5) + 8 * u;
+            vr[u] = load4<VEC>(a.v + (size_t)(t0 + min(s, n - 1)) * a.v_stride + (size_t)h * dv, (tid & 31) * 4, dv, s < n);
         }
     }
-    if (tid < GC) {
-        const size_t th = (size_t)(t0 + tid) * a.heads + h;
-        const float ld = tid < n ? a.log_decay[th] : 0.0f;
-        bt[tid] = tid < n ? a.beta[th] : 0.0f;
-        // inclusive prefix sum of log decay over the chunk (one wave)
-        float g = ld;
+    // Inclusive prefix sum of log decay over the chunk (lane: token).
+    float gl = lane < n ? ld_raw : 0.0f;
 #pragma unroll
-        for (int o = 1; o < 64; o <<= 1) {
-            const float up = __shfl_up(g, o);
-            if (tid >= (uint32_t)o) g += up;
-        }
-        G[tid] = g;
+    for (int o = 1; o < 64; o <<= 1) {
+        const float up = __shfl_up(gl, o);
+        if (lane >= (uint32_t)o) gl += up;
     }
-    __syncthreads();
-    // The lower 16 x 16 tiles of K K^T and Q K^T on MFMA: 10 tiles each,
-    // (sb, rb) with rb <= sb, five per wave; the upper tiles of A are zero.
+    // The largest exp(G_C - G_r) (1 when no decay exceeds one).
+    const float gc = __shfl(gl, 63);
+    float emax = gc - gl;
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) emax = fmaxf(emax, __shfl_xor(emax, o));
+    const int ek = exponent_of(expf(emax));
+    if (w == 0) {
+        G[lane] = gl;
+        bt[lane] = lane < n ? bt_raw : 0.0f;
+    }
     {
-        const uint32_t lane = tid & 63, w = tid >> 6, m16 = lane & 15, kq = lane >> 4;
-        gv4f acc[5];
+        float sq = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 5; u++) {
-            const uint32_t t = w + 4 * u, l = t % 10;
-            const uint32_t sb = l >= 6 ? 3 : (l >= 3 ? 2 : (l >= 1 ? 1 : 0));
-            const uint32_t rb = l - sb * (sb + 1) / 2;
-            acc[u] = tile_kk<GKD, SPAD, SPAD>((t < 10 ? kh : qh) + 16 * sb * SPAD, kh + 16 * rb * SPAD,
-                                              (gv4f){0, 0, 0, 0}, lane);
+        for (int u = 0; u < 8; u++) {
+            sq += (kr[u][0] * kr[u][0] + kr[u][1] * kr[u][1]) + (kr[u][2] * kr[u][2] + kr[u][3] * kr[u][3]);
+            *(gv4f *)(kh + own * SPAD + 16 * u + 4 * g) = kr[u];
         }
-        float *Aout = a.norms + ((size_t)h * nch + c) * ctox_gdn_chunk_floats() + GC * GC;
-        __syncthreads();  // every tile has read q^: its rows become M
+        sq = groups_sum(sq);
+        if (g == 0) kinv_s[own] = own < n ? 1.0f / sqrtf(sq + 1e-6f) : 0.0f;
+    }
+    float qinv;
+    {   // Q fragments of strip w: normalised rows
+        float sq = 0.0f;
 #pragma unroll
-        for (int u = 0; u < 5; u++) {
-            const uint32_t t = w + 4 * u, l = t % 10;
-            const uint32_t sb = l >= 6 ? 3 : (l >= 3 ? 2 : (l >= 1 ? 1 : 0));
-            const uint32_t rb = l - sb * (sb + 1) / 2;
+        for (int u = 0; u < 8; u++)
+            sq += (qr[u][0] * qr[u][0] + qr[u][1] * qr[u][1]) + (qr[u][2] * qr[u][2] + qr[u][3] * qr[u][3]);
+        qinv = own < n ? 1.0f / sqrtf(groups_sum(sq) + 1e-6f) : 0.0f;
+        const float sc = qinv * 16384.0f;
+        uint4 *dst = (uint4 *)(base + GF_Q) + w * 512 + lane;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            uint4 f[2];
+            split8(qr[2 * st] * sc, qr[2 * st + 1] * sc, f);
+            dst[128 * st] = f[0];
+            dst[128 * st + 64] = f[1];
+        }
+    }
+    lds_barrier();
+    if (w == 0) ekf[lane] = expf(gc - gl) * kinv_s[lane] * pow2(14 - ek);
+    // 16 x 16 tiles on the raw rows, scaled by the inverse norms afterwards,
+    // five per wave: K Q^T of token strip w (rows r, columns t: the result is
+    // A's fragment order) and K K^T of strip 3 - w.
+    gv4f acc[5];
+    const float *krow = kh + m16 * SPAD + 4 * g;
+#pragma unroll
+    for (uint32_t u = 0; u < 4; u++)
+        if (u <= w) acc[u] = tile_rows(krow + 16 * u * SPAD, qr);
+    {
+        gv4f ks[8];  // strip 3 - w as the right operand
+#pragma unroll
+        for (int u = 0; u < 8; u++) ks[u] = *(const gv4f *)(krow + 16 * (3 - w) * SPAD + 16 * u);
+#pragma unroll
+        for (uint32_t u = 1; u < 5; u++)
+            if (u > w) acc[u] = tile_rows(krow + 16 * (u - w - 1) * SPAD, ks);
+    }
+    {   // A: row t = own, this lane's r = 16 u + 4 g + x
+        float sq = 0.0f;
+#pragma unroll
+        for (uint32_t u = 0; u < 4; u++) {
+            if (u > w) continue;
 #pragma unroll
             for (int x = 0; x < 4; x++) {
-                const uint32_t s = 16 * sb + 4 * kq + x, r = 16 * rb + m16;
-                const float dec = expf(G[s] - G[r]) * kinv_s[r] * (t < 10 ? kinv_s[s] : qinv_s[s] * qscale);
-                if (t < 10) mm[s * TPAD + r] = r < s ? dec * acc[u][x] : 0.0f;
-                else Aout[s * GC + r] = r <= s ? dec * acc[u][x] : 0.0f;
+                const uint32_t r = 16 * u + 4 * g + x;
+                const float val = r <= own ? expf(G[own] - G[r]) * (kinv_s[r] * qinv) * acc[u][x] : 0.0f;
+                acc[u][x] = val;
+                sq += val * val;
             }
         }
-        for (uint32_t e = tid; e < GC * GC / 4; e += 256) {
-            const uint32_t s = e / 16, r = (e % 16) * 4;
-            if (r / 16 > s / 16) *(float4 *)(Aout + s * GC + r) = make_float4(0, 0, 0, 0);
+        const int e = exponent_of(sqrtf(groups_sum(sq)));
+        const float sc = pow2(14 - e);
+        if (g == 0) aux[128 + own] = qscale * pow2(e - 14);
+        uint4 *dst = (uint4 *)(base + GF_A) + w * 256 + lane;
+        const gv4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
+        uint4 f[2];
+        split8(acc[0] * sc, w >= 1 ? acc[1] * sc : zero, f);
+        dst[0] = f[0];
+        dst[64] = f[1];
+        split8(w >= 2 ? acc[2] * sc : zero, w >= 3 ? acc[3] * sc : zero, f);
+        dst[128] = f[0];
+        dst[192] = f[1];
+    }
+    {   // L of strip 3 - w, strictly lower: the tile's rows are r, its columns s
+        const uint32_t s = 16 * (3 - w) + m16;
+        const float f = bt[s] * kinv_s[s];
+#pragma unroll
+        for (uint32_t u = 1; u < 5; u++) {
+            if (u <= w) continue;
+#pragma unroll
+            for (int x = 0; x < 4; x++) {
+                const uint32_t r = 16 * (u - w - 1) + 4 * g + x;
+                tt[s * TPAD + r] = r < s ? f * kinv_s[r] * acc[u][x] : 0.0f;
+            }
         }
     }
-    __syncthreads();
-    float *base = a.norms + ((size_t)h * nch + c) * ctox_gdn_chunk_floats();
-    // T = (I + L)^{-1}, L = diag(b) M strictly lower, blockwise over 16 x 16
-    // blocks into LDS (tt, over the k rows, free after the tiles):
-    //   T_ii = (I + L_ii)^{-1}                   forward substitution, wave i;
+    lds_barrier();
+    // T0 = (I + L)^{-1} over L, blockwise over 16 x 16 blocks:
+    //   T_ii = (I + L_ii)^{-1}                   forward substitution, wave i
+    //                                            (row s of L is last read for row s of T);
     //   T_ij = -T_ii sum_{k=j}^{i-1} L_ik T_kj   block row i after row i - 1,
     //                                            task j on wave j, on MFMA.
-    float *tt = kh;
-    {
-        const uint32_t lane = tid & 63, w = tid >> 6, m16 = lane & 15, kq = lane >> 4;
-        if (lane < 16) {
-            const uint32_t cc = 16 * w + lane;
-            float col[16];
+    if (lane < 16) {
+        float *blk = tt + 16 * w * TPAD + 16 * w;
+        float col[16];
 #pragma unroll
-            for (int s = 0; s < 16; s++) {
-                const uint32_t row = 16 * w + s;
-                float acc = 0.0f;
+        for (int s = 0; s < 16; s++) {
+            float sum = 0.0f;
 #pragma unroll
-                for (int r = 0; r < s; r++) acc = fmaf(mm[row * TPAD + 16 * w + r], col[r], acc);
-                col[s] = ((uint32_t)s == lane ? 1.0f : 0.0f) - bt[row] * acc;
-                tt[row * TPAD + cc] = col[s];
-            }
+            for (int r = 0; r < s; r++) sum = fmaf(blk[s * TPAD + r], col[r], sum);
+            col[s] = ((uint32_t)s == lane ? 1.0f : 0.0f) - sum;
         }
 #pragma unroll
-        for (uint32_t bi = 1; bi < 4; bi++) {
-            __syncthreads();  // block row bi - 1 (and the diagonal) written
-            if (w < bi) {
-                const uint32_t bj = w;
-                // X = sum_k L_ik T_kj: A = L rows of block bi, B = T rows of block k.
-                gv4f x = {0.0f, 0.0f, 0.0f, 0.0f};
-                for (uint32_t bk = bj; bk < bi; bk++) {
-                    const float b = bt[16 * bi + m16];
-#pragma unroll
-                    for (int u = 0; u < 4; u++) {
-                        const uint32_t kk = 16 * bk + 4 * u + kq;
-                        x = mfma4(b * mm[(16 * bi + m16) * TPAD + kk], tt[kk * TPAD + 16 * bj + m16], x);
-                    }
-                }
-                // T_ij = -T_ii X. Lane (kq, n) holds X rows 4 kq + u of column
-                // n, so MFMA u takes k = 4 kq + u: A reads T_ii[m][4 kq + u].
-                gv4f y = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int u = 0; u < 4; u++)
-                    y = mfma4(tt[(16 * bi + m16) * TPAD + 16 * bi + 4 * kq + u], x[u], y);
-#pragma unroll
-                for (int u = 0; u < 4; u++) tt[(16 * bi + 4 * kq + u) * TPAD + 16 * bj + m16] = -y[u];
-            }
-        }
-        __syncthreads();
-        for (uint32_t e = tid; e < GC * GC / 4; e += 256) {
-            const uint32_t s = e / 16, r = (e % 16) * 4;
-            const bool up = r / 16 > s / 16;
-            *(float4 *)(base + s * GC + r) = up ? make_float4(0, 0, 0, 0)
-                                                : make_float4(tt[s * TPAD + r], tt[s * TPAD + r + 1],
-                                                              tt[s * TPAD + r + 2], tt[s * TPAD + r + 3]);
-        }
+        for (int s = 0; s < 16; s++) blk[s * TPAD + lane] = col[s];
     }
-    if (tid < GC) {
-        const float g = expf(G[tid]);
-        base[2 * GC * GC + tid] = g;
-        base[2 * GC * GC + GC + tid] = expf(G[GC - 1] - G[tid]);
-        base[2 * GC * GC + 2 * GC + tid] = kinv_s[tid];
-        base[2 * GC * GC + 3 * GC + tid] = qinv_s[tid] * qscale * g;
-    }
-}
-
-// A buffer resource over [p, p + bytes) whose fields the compiler keeps in
-// scalar registers: p and bytes are wave-uniform but computed through vector
-// registers, and a resource in vector registers costs a waterfall loop per load.
-__device__ __forceinline__ __amdgpu_buffer_rsrc_t uniform_rsrc(const void *p, uint32_t bytes) {
-    const uint64_t v = (uint64_t)p;
-    const uint64_t u = ((uint64_t)__builtin_amdgcn_readfirstlane((uint32_t)(v >> 32)) << 32) |
-                       (uint32_t)__builtin_amdgcn_readfirstlane((uint32_t)v);
-    return __builtin_amdgcn_make_buffer_rsrc((void *)u, (short)0, (int)__builtin_amdgcn_readfirstlane(bytes), 0x00020000);
-}
-
-// Registers holding the next chunk while the current one computes.
-struct GdnPrefetch {
-    float4 k[8], q[8];   // 64 x 128 each: float4 index tid + 256 m
-    float4 t[4], am[4];  // T, A: 64 x 64 each
-    float4 v;            // 64 x 16 value slice: row tid / 4, part tid % 4
-    float4 aux;          // g / g_C/g / kinv / q scale (threads 0..63), float4 tid % 16 of array tid / 16
-    float beta;          // threads 0..63
-};
-
-// VEC: key_dim and value_dim multiples of 4 and 16, token strides multiples
-// of 4 floats, q, k, v 16-byte aligned and a chunk's rows spanning under
-// 2 GB; the host launches the VEC instantiation exactly then. Its loads are
-// 16-byte buffer reads with no branches (the generic path's predicated reads
-// make the compiler wait for every outstanding load at each branch join,
-// which serialises the next chunk's prefetch).
-template <bool VEC>
-__device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
-    // k^ rows [s][i]; (g q^) rows [s][i]; T [s][r]; A [t][r]; S^T [n][i] (x2);
-    // Y^T / D^T [n][s]; (b v)^T [n][s]; D [r][n] for the state update; K~^T [i][r].
-    __shared__ __align__(16) float kh[GC * SPAD];
-    __shared__ __align__(16) float qh[GC * SPAD];
-    __shared__ __align__(16) float tm[GC * TSPAD];
-    __shared__ __align__(16) float am[GC * TSPAD];
-    __shared__ __align__(16) float st[2][GVS * SPAD];
-    __shared__ __align__(16) float yt[GVS * TSPAD];
-    __shared__ __align__(16) float vt[GVS * TSPAD];
-    __shared__ float eg[GC], ec[GC], kinv[GC], qsc[GC], bt[GC];
-    const uint32_t tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
-    const uint32_t m16 = lane & 15, kq = lane >> 4;
-    const uint32_t slices = (a.value_dim + GVS - 1) / GVS;
-    // Workgroup b runs on XCD b % 8. All slices of one head are placed on the
-    // same XCD so that they share the chunk's k, q, T and A in that XCD's L2:
-    // XCD x takes heads x, x + 8, ..., its q-th workgroup being slice q % slices
-    // of head x + 8 (q / slices). The grid is 8 * ceil(heads / 8) * slices.
-    const uint32_t xcd = blockIdx.x & 7, qx = blockIdx.x >> 3;
-    const uint32_t h = xcd + 8 * (qx / slices), j0 = (qx % slices) * GVS;
-    if (h >= a.heads) return;
-    const uint32_t nch = (a.tokens + a.chunk - 1) / a.chunk;
-    const uint32_t dk = a.key_dim, dv = a.value_dim;
-    const size_t rowv = (size_t)a.heads * dv;
-    float *S = a.state + (size_t)h * dk * dv;
-    for (uint32_t e = tid; e < GKD * GVS; e += 256) {
-        const uint32_t i = e / GVS, n = e % GVS;
-        st[0][n * SPAD + i] = (i < dk && j0 + n < dv) ? S[(size_t)i * dv + j0 + n] : 0.0f;
-    }
-
-    // parts: 1 = k (with q on the generic path), 2 = q, 4 = T, A, v, aux, beta.
-    auto fetch = [&](GdnPrefetch &p, uint32_t c, const int parts) {
-        const uint32_t t0 = c * a.chunk, n = min(a.chunk, a.tokens - t0);
-        const float *base = a.norms + ((size_t)h * nch + c) * ctox_gdn_chunk_floats();
-        // Branch-free loads: one buffer over the chunk's rows of this key head
-        // (of this value slice); a lane past the chunk or past key_dim reads at
-        // the buffer's end, which the range check returns as zero.
-        const uint32_t kq_end = VEC ? ((n - 1) * a.qk_stride + dk) * 4 : 0;
-        const size_t kq0 = (size_t)t0 * a.qk_stride + (size_t)(h / a.rep) * dk;
-        const __amdgpu_buffer_rsrc_t rk = uniform_rsrc(a.k + kq0, kq_end);
-        const __amdgpu_buffer_rsrc_t rq = uniform_rsrc(a.q + kq0, kq_end);
+    {   // K^T fragments of key tiles 2 w, 2 w + 1, with the decay to the chunk's end
+        uint4 *dst = (uint4 *)(base + GF_K) + w * 512 + lane;
 #pragma unroll
-        for (int m = 0; m < 8; m++) {
-            const uint32_t f = tid + 256 * m, s = f >> 5, i = (f & 31) * 4;
-            const bool ok = s < n && i < dk;
-            if (VEC) {
-                const uint32_t off = ok ? (s * a.qk_stride + i) * 4 : kq_end;
-                if (parts & 1) p.k[m] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rk, off, 0, 0));
-                if (parts & 2) p.q[m] = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rq, off, 0, 0));
-            } else if (parts & 1) {
-                const size_t off = (size_t)(t0 + (ok ? s : 0)) * a.qk_stride + (size_t)(h / a.rep) * dk + (ok ? i : 0);
-                float kk4[4], qq4[4];
+        for (int t = 0; t < 2; t++) {
+            const float *kp = kh + 16 * (2 * w + t) + m16;
+#pragma unroll
+            for (int st = 0; st < 2; st++) {
+                gv4f lo, up;
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
-                    const bool ox = s < n && i + x < dk;
-                    kk4[x] = ox ? a.k[off + x] : 0.0f;
-                    qq4[x] = ox ? a.q[off + x] : 0.0f;
+                    const uint32_t r = 32 * st + 4 * g + x;
+                    lo[x] = kp[r * SPAD] * ekf[r];
+                    up[x] = kp[(r + 16) * SPAD] * ekf[r + 16];
                 }
-                p.k[m] = make_float4(kk4[0], kk4[1], kk4[2], kk4[3]);
-                p.q[m] = make_float4(qq4[0], qq4[1], qq4[2], qq4[3]);
+                uint4 f[2];
+                split8(lo, up, f);
+                dst[256 * t + 128 * st] = f[0];
+                dst[256 * t + 128 * st + 64] = f[1];
             }
         }
-        if (!(parts & 4)) return;
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            p.t[m] = ((const float4 *)base)[tid + 256 * m];
-            p.am[m] = ((const float4 *)(base + GC * GC))[tid + 256 * m];
-        }
-        {
-            const uint32_t s = tid >> 2, part = tid & 3;
-            const bool ok = s < n;
-            if (VEC) {
-                const uint32_t v_end = ((n - 1) * a.v_stride + GVS) * 4;
-                const __amdgpu_buffer_rsrc_t rv = uniform_rsrc(a.v + (size_t)t0 * a.v_stride + (size_t)h * dv + j0, v_end);
-                p.v = __builtin_bit_cast(float4, __builtin_amdgcn_raw_buffer_load_b128(rv, ok ? (s * a.v_stride + 4 * part) * 4 : v_end, 0, 0));
-            } else {
-                const size_t off = (size_t)(t0 + (ok ? s : 0)) * a.v_stride + (size_t)h * dv + j0 + 4 * part;
-                float v4[4];
-#pragma unroll
-                for (int x = 0; x < 4; x++) v4[x] = (ok && j0 + 4 * part + x < dv) ? a.v[off + x] : 0.0f;
-                p.v = make_float4(v4[0], v4[1], v4[2], v4[3]);
-            }
-        }
-        p.aux = tid < 64 ? ((const float4 *)(base + 2 * GC * GC))[tid] : make_float4(0, 0, 0, 0);
-        {
-            const uint32_t b_end = ((n - 1) * a.heads + 1) * 4;
-            const __amdgpu_buffer_rsrc_t rb = uniform_rsrc(a.beta + (size_t)t0 * a.heads + h, b_end);
-            p.beta = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rb, tid < n ? tid * a.heads * 4 : b_end, 0, 0));
-        }
-    };
-
-    GdnPrefetch pf;
-    fetch(pf, 0, 7);
-    uint32_t cur = 0;
-    for (uint32_t c = 0; c < nch; c++) {
-        const uint32_t t0 = c * a.chunk, n = min(a.chunk, a.tokens - t0);
-        lds_barrier();  // the previous chunk is done with every buffer
-        if (tid < GC) {
-            float *aux = tid < 16 ? eg : (tid < 32 ? ec : (tid < 48 ? kinv : qsc));
-            ((float4 *)aux)[tid & 15] = pf.aux;
-            bt[tid] = pf.beta;
-        }
-        lds_barrier();
-        // Stage: k^ = k kinv; (g q^) = q qinv qscale exp(G) (one factor from
-        // the prep); T; A; (b v)^T.
-#pragma unroll
-        for (int m = 0; m < 8; m++) {
-            const uint32_t f = tid + 256 * m, s = f >> 5, i = (f & 31) * 4;
-            const float ks = kinv[s], qs = qsc[s];
-            *(float4 *)(kh + s * SPAD + i) = make_float4(pf.k[m].x * ks, pf.k[m].y * ks, pf.k[m].z * ks, pf.k[m].w * ks);
-            *(float4 *)(qh + s * SPAD + i) = make_float4(pf.q[m].x * qs, pf.q[m].y * qs, pf.q[m].z * qs, pf.q[m].w * qs);
-        }
-#pragma unroll
-        for (int m = 0; m < 4; m++) {
-            const uint32_t f = tid + 256 * m, s = f >> 4, r = (f & 15) * 4;
-            *(float4 *)(tm + s * TSPAD + r) = pf.t[m];
-            *(float4 *)(am + s * TSPAD + r) = pf.am[m];
-        }
-        {
-            const uint32_t s = tid >> 2, part = tid & 3;
-            const float b = bt[s];
-            vt[(4 * part + 0) * TSPAD + s] = pf.v.x * b;
-            vt[(4 * part + 1) * TSPAD + s] = pf.v.y * b;
-            vt[(4 * part + 2) * TSPAD + s] = pf.v.z * b;
-            vt[(4 * part + 3) * TSPAD + s] = pf.v.w * b;
-        }
-        lds_barrier();
-        // The next chunk's loads are issued in three groups between this
-        // chunk's products, so that their address traffic overlaps MFMA work;
-        // the loop's barriers order LDS only, so nothing waits for them before
-        // the next chunk's staging.
-        const bool more = c + 1 < nch;
-        if (more) fetch(pf, c + 1, 4);
-        const float *Sc = st[cur];
-        // Y^T[n][s] = (b v)^T - b_s g_s (K S)[s][n]   (wave w: rows s = 16w..16w+15)
-        {
-            gv4f acc = tile_kk<GKD, SPAD, SPAD>(kh + 16 * w * SPAD, Sc, (gv4f){0, 0, 0, 0}, lane);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const uint32_t s = 16 * w + 4 * kq + r;
-                yt[m16 * TSPAD + s] = vt[m16 * TSPAD + s] - bt[s] * eg[s] * acc[r];
-            }
-        }
-        if (more) fetch(pf, c + 1, 1);
-        lds_barrier();
-        // D = T Y  (T rows [s][r] and Y^T [n][r] are both r-contiguous)
-        gv4f dacc = tile_kk<GC, TSPAD, TSPAD>(tm + 16 * w * TSPAD, yt, (gv4f){0, 0, 0, 0}, lane);
-        lds_barrier();
-        // D^T [n][s] into yt, and (D^T scaled by g_C / g_s) into vt, whose
-        // (b v)^T the Y step has consumed: the state update's left operand.
-#pragma unroll
-        for (int r = 0; r < 4; r++) {
-            const uint32_t s = 16 * w + 4 * kq + r;
-            yt[m16 * TSPAD + s] = dacc[r];
-            vt[m16 * TSPAD + s] = dacc[r] * ec[s];
-        }
-        lds_barrier();
-        if (more) fetch(pf, c + 1, 2);
-        // O = (g Q) S + A D
-        {
-            gv4f acc = tile_kk<GKD, SPAD, SPAD>(qh + 16 * w * SPAD, Sc, (gv4f){0, 0, 0, 0}, lane);
-            acc = tile_kk<GC, TSPAD, TSPAD>(am + 16 * w * TSPAD, yt, acc, lane);
-#pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const uint32_t s = 16 * w + 4 * kq + r, j = j0 + m16;
-                if (s < n && j < dv) a.out[(size_t)(t0 + s) * rowv + (size_t)h * dv + j] = acc[r];
-            }
-        }
-        // S'^T[n][i] = g_C S^T[n][i] + sum_r D^T[n][r] exp(G_C - G_r) k^[r][i]
-        //   as a 16 x 16 tile per (n, i-block): A = the scaled D^T [n][r]
-        //   (r-contiguous), B = k^[r][i] read column-wise.
-        {
-            const float decC = eg[GC - 1];
-            float *Sn = st[cur ^ 1];
-#pragma unroll
-            for (int half = 0; half < 2; half++) {
-                const uint32_t i0 = 32 * w + 16 * half;
-                gv4f acc;
-#pragma unroll
-                for (int r = 0; r < 4; r++) acc[r] = decC * Sc[(4 * kq + r) * SPAD + i0 + m16];
-                const float *ap = vt + m16 * TSPAD + kq * (GC / 4);
-                gv4f c1 = {0.0f, 0.0f, 0.0f, 0.0f};
-#pragma unroll
-                for (int u = 0; u < GC / 4; u += 2) {
-                    const uint32_t rr = kq * (GC / 4) + u;
-                    acc = mfma4(ap[u], kh[rr * SPAD + i0 + m16], acc);
-                    c1 = mfma4(ap[u + 1], kh[(rr + 1) * SPAD + i0 + m16], c1);
-                }
-                acc += c1;
-                // acc rows = n (4 kq + r), columns = i0 + m16
-#pragma unroll
-                for (int r = 0; r < 4; r++) Sn[(4 * kq + r) * SPAD + i0 + m16] = acc[r];
-            }
-        }
-        cur ^= 1;
     }
-    __syncthreads();
-    for (uint32_t e = tid; e < GKD * GVS; e += 256) {
-        const uint32_t i = e / GVS, n = e % GVS;
-        if (i < dk && j0 + n < dv) S[(size_t)i * dv + j0 + n] = st[cur][n * SPAD + i];
+#pragma unroll
+    for (uint32_t bi = 1; bi < 4; bi++) {
+        lds_barrier();  // block row bi - 1 (and the diagonal) written
+        // X = sum_k L_ik T_kj: A = L rows of block bi, B = T rows of block k.
+        gv4f y = {0.0f, 0.0f, 0.0f, 0.0f};
+        if (w < bi) {
+            gv4f x = y;
+            for (uint32_t bk = w; bk < bi; bk++) {
+#pragma unroll
+                for (int u = 0; u < 4; u++) {
+                    const uint32_t kk = 16 * bk + 4 * u + g;
+                    x = mfma4(tt[(16 * bi + m16) * TPAD + kk], tt[kk * TPAD + 16 * w + m16], x);
+                }
+            }
+            // T_ij = -T_ii X. Lane (g, n) holds X rows 4 g + u of column n, so
+            // MFMA u takes k = 4 g + u: A reads T_ii[m][4 g + u].
+#pragma unroll
+            for (int u = 0; u < 4; u++) y = mfma4(tt[(16 * bi + m16) * TPAD + 16 * bi + 4 * g + u], x[u], y);
+        }
+        lds_barrier();  // block row bi of L is dead
+        if (w < bi) {
+#pragma unroll
+            for (int u = 0; u < 4; u++) tt[(16 * bi + 4 * g + u) * TPAD + 16 * w + m16] = -y[u];
+        }
+    }
+    lds_barrier();
+    // tt: T0 diag(b kinv) (W's left operand, on the raw K rows); in registers,
+    // for tt later: the decayed T0 diag(b) (U's). Lane: column r, rows 16 w + i.
+    // Blocks above the diagonal are read by no product.
+    float tu[16];
+    {
+        const float b = bt[lane], ki = kinv_s[lane];
+#pragma unroll
+        for (int i = 0; i < 16; i++) {
+            const uint32_t s = 16 * w + i;
+            const float t = tt[s * TPAD + lane] * b;
+            tu[i] = lane <= s ? t * expf(G[s] - gl) : 0.0f;
+            tt[s * TPAD + lane] = t * ki;
+        }
+    }
+    lds_barrier();
+    // W^T of key tiles 2 w, 2 w + 1 (rows i, columns s: W's fragment order).
+    gv4f wt[4][2];
+#pragma unroll
+    for (int st = 0; st < 4; st++) wt[st][0] = wt[st][1] = gv4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int rb = 0; rb < 4; rb++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t r = 16 * rb + 4 * u + g;
+            const float a0 = kh[r * SPAD + 32 * w + m16], a1 = kh[r * SPAD + 32 * w + 16 + m16];
+#pragma unroll
+            for (int st = rb; st < 4; st++) {
+                const float b = tt[(16 * st + m16) * TPAD + r];
+                wt[st][0] = mfma4(a0, b, wt[st][0]);
+                wt[st][1] = mfma4(a1, b, wt[st][1]);
+            }
+        }
+#pragma unroll
+    for (int st = 0; st < 4; st++) {
+        float sq = 0.0f;
+#pragma unroll
+        for (int x = 0; x < 4; x++) sq += wt[st][0][x] * wt[st][0][x] + wt[st][1][x] * wt[st][1][x];
+        sq = groups_sum(sq);
+        if (g == 0) wsq[w][16 * st + m16] = sq;
+    }
+    lds_barrier();  // K rows and W's left operand are dead
+#pragma unroll
+    for (int i = 0; i < 16; i++) tt[(16 * w + i) * TPAD + lane] = tu[i];
+#pragma unroll
+    for (int u = 0; u < 8; u++) *(gv4f *)(kh + ((tid >> 5) + 8 * u) * SPAD + (tid & 31) * 4) = vr[u];
+    {
+        uint4 *dst = (uint4 *)(base + GF_W) + 128 * w + lane;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            const uint32_t s = 16 * st + m16;
+            const int e = exponent_of(sqrtf((wsq[0][s] + wsq[1][s]) + (wsq[2][s] + wsq[3][s])));
+            const float sc = pow2(14 - e);
+            uint4 f[2];
+            split8(wt[st][0] * sc, wt[st][1] * sc, f);
+            dst[512 * st] = f[0];
+            dst[512 * st + 64] = f[1];
+        }
+    }
+    if (w == 0) {
+        const float ge = expf(gl);
+        const float nw = sqrtf((wsq[0][lane] + wsq[1][lane]) + (wsq[2][lane] + wsq[3][lane]));
+        aux[lane] = ge * pow2(exponent_of(nw) - 14);
+        aux[64 + lane] = qscale * ge * pow2(-14);
+        float wn = ge * nw;
+#pragma unroll
+        for (int o = 32; o > 0; o >>= 1) wn = fmaxf(wn, __shfl_xor(wn, o));
+        if (lane == GC - 1) {
+            aux[320] = ge;
+            aux[321] = pow2(ek - 14);
+            aux[322] = wn;
+        }
+    }
+    lds_barrier();
+    // U of value tiles 2 w, 2 w + 1 and its largest magnitude per column.
+    if (32 * w >= dv) return;
+    gv4f us[4][2];
+#pragma unroll
+    for (int st = 0; st < 4; st++) us[st][0] = us[st][1] = gv4f{0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+    for (int rb = 0; rb < 4; rb++)
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            const uint32_t r = 16 * rb + 4 * u + g;
+            const float v0 = kh[r * SPAD + 32 * w + m16], v1 = kh[r * SPAD + 32 * w + 16 + m16];
+#pragma unroll
+            for (int st = rb; st < 4; st++) {
+                const float t = tt[(16 * st + m16) * TPAD + r];
+                us[st][0] = mfma4(t, v0, us[st][0]);
+                us[st][1] = mfma4(t, v1, us[st][1]);
+            }
+        }
+    float4 *dst = (float4 *)(base + GF_U) + 512 * w + lane;
+#pragma unroll
+    for (int j = 0; j < 2; j++) {
+        float mx = 0.0f;
+#pragma unroll
+        for (int st = 0; st < 4; st++) {
+            const gv4f x = us[st][j];
+            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
+            dst[256 * j + 64 * st] = make_float4(x[0], x[1], x[2], x[3]);
+        }
+        mx = groups_max(mx);
+        if (g == 0) aux[192 + 16 * (2 * w + j) + m16] = mx;
     }
 }
 
-extern "C" __global__ __launch_bounds__(256) void ctox_gdn_chunk_scan_gfx950(GdnArgs a) { chunk_scan<false>(a); }
-extern "C" __global__ __launch_bounds__(256) void ctox_gdn_chunk_scan_vec_gfx950(GdnArgs a) { chunk_scan<true>(a); }
+// A chunk's operands of one wave, in registers one chunk ahead.
+template <int NT>
+struct GdnStateOps {     // waves 0..3
+    uint4 w[4][2];       // W strip, key steps
+    uint4 k[2][2][2];    // K^T key tiles 2 w, 2 w + 1, token steps
+    float4 u[NT], fw;
+    float mu[NT], gc, fk, wn;
+};
+template <int NT>
+struct GdnOutOps {       // waves 4..7
+    uint4 q[4][2];
+    uint4 am[2][2];
+    float4 fq, fa;
+    float mu[NT], wn;
+};
+
+// The operands' exchange. One buffer each: state operands are read between the
+// first barrier of a chunk and its second, D's after it.
+template <int NT>
+struct GdnScanLds {
+    uint4 s[NT][4][2][64];    // [value tile][key step][hi, lo][lane]
+    uint4 d[NT][2][2][64];    // [value tile][token step][hi, lo][lane]; a strip is half of each 16 B
+    float sf[NT][4][16];      // [value tile][key step][column]: what the state operand was divided by
+};
+
+// X = (rows) x S_0 with the key steps' column factors applied.
+template <int NT>
+__device__ __forceinline__ gv4f times_state(const uint4 (&x)[4][2], const GdnScanLds<NT> &L, int j, uint32_t lane,
+                                            const float (&sf)[4]) {
+    gv4f acc[4];
+#pragma unroll
+    for (int k = 0; k < 4; k++) {
+        const uint4 s[2] = {L.s[j][k][0][lane], L.s[j][k][1][lane]};
+        acc[k] = mfma_split(x[k], s, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+    }
+    return (acc[0] * sf[0] + acc[1] * sf[1]) + (acc[2] * sf[2] + acc[3] * sf[3]);
+}
+
+// Exponent of D's scale: |D| <= max|U| + max_s |g_s W_s| |S column|, and a
+// key step's 32 values are below sf 2^15 each.
+__device__ __forceinline__ int d_exponent(float mu, float wn, const float (&sf)[4]) {
+    return exponent_of(mu + wn * (32768.0f * 5.66f) * ((sf[0] + sf[1]) + (sf[2] + sf[3])));
+}
+
+// NT: value tiles (of 16 columns) per workgroup.
+template <int NT>
+__device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
+    __shared__ GdnScanLds<NT> L;
+    const uint32_t tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const uint32_t m16 = lane & 15, g = lane >> 4, w = wave & 3;
+    const uint32_t slices = (a.value_dim + 16 * NT - 1) / (16 * NT);
+    uint32_t h, slice;
+    head_of_block(blockIdx.x, slices, h, slice);
+    if (h >= a.heads) return;
+    const uint32_t dk = a.key_dim, dv = a.value_dim, nch = a.chunks, j0 = slice * 16 * NT;
+    const char *scratch = (const char *)a.norms + (size_t)h * nch * CTOX_GDN_CHUNK_BYTES;
+    const bool second = a.chunk > 32;  // tokens in the second step
+
+    if (wave < 4) {
+        auto load = [&](GdnStateOps<NT> &p, uint32_t c) {
+            const char *b = scratch + (size_t)min(c, nch - 1) * CTOX_GDN_CHUNK_BYTES;
+            const uint4 *wp = (const uint4 *)(b + GF_W) + 512 * w + lane, *kp = (const uint4 *)(b + GF_K) + 512 * w + lane;
+            const float4 *up = (const float4 *)(b + GF_U) + 256 * (NT * slice) + 64 * w + lane;
+            const float *aux = (const float *)(b + GF_AUX);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int x = 0; x < 2; x++) p.w[k][x] = wp[128 * k + 64 * x];
+#pragma unroll
+            for (int j = 0; j < NT; j++) p.u[j] = up[256 * j];
+            p.fw = *(const float4 *)(aux + 16 * w + 4 * g);
+#pragma unroll
+            for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
+            p.wn = aux[322];
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int u = 0; u < 2; u++)
+#pragma unroll
+                    for (int x = 0; x < 2; x++) p.k[t][u][x] = kp[256 * t + 128 * u + 64 * x];
+            p.gc = aux[320];
+            p.fk = aux[321];
+        };
+        // State rows 32 w + 16 t + 4 g + r, column j0 + 16 j + m16.
+        gv4f st[NT][2];
+        float *S = a.state + (size_t)h * dk * dv;
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    // (no branch around the load: they are all in flight at once)
+                    const uint32_t i = 32 * w + 16 * t + 4 * g + r, col = j0 + 16 * j + m16;
+                    const float x = S[(size_t)min(i, dk - 1) * dv + min(col, dv - 1)];
+                    st[j][t][r] = i < dk && col < dv ? x : 0.0f;
+                }
+        auto publish = [&](int j) {
+            float mx = 0.0f;
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) mx = fmaxf(mx, fabsf(st[j][t][r]));
+            const int e = exponent_of(groups_max(mx));
+            const float sc = pow2(15 - e);
+            uint4 f[2];
+            split8(st[j][0] * sc, st[j][1] * sc, f);
+            L.s[j][w][0][lane] = f[0];
+            L.s[j][w][1][lane] = f[1];
+            if (g == 0) L.sf[j][w][m16] = pow2(e - 15);
+        };
+        auto step = [&](const GdnStateOps<NT> &p) {
+            float fd[NT];
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const float sf[4] = {L.sf[j][0][m16], L.sf[j][1][m16], L.sf[j][2][m16], L.sf[j][3][m16]};
+                const gv4f x = times_state<NT>(p.w, L, j, lane, sf);
+                const int e = d_exponent(p.mu[j], p.wn, sf);
+                const float sc = pow2(15 - e);
+                fd[j] = pow2(e - 15);
+                uint2 hi, lo;
+                split2((p.u[j].x - p.fw.x * x[0]) * sc, (p.u[j].y - p.fw.y * x[1]) * sc, hi.x, lo.x);
+                split2((p.u[j].z - p.fw.z * x[2]) * sc, (p.u[j].w - p.fw.w * x[3]) * sc, hi.y, lo.y);
+                ((uint2 *)&L.d[j][w >> 1][0][lane])[w & 1] = hi;
+                ((uint2 *)&L.d[j][w >> 1][1][lane])[w & 1] = lo;
+            }
+            lds_barrier();
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const uint4 d0[2] = {L.d[j][0][0][lane], L.d[j][0][1][lane]};
+                gv4f n0 = mfma_split(p.k[0][0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+                gv4f n1 = mfma_split(p.k[1][0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+                if (second) {
+                    const uint4 d1[2] = {L.d[j][1][0][lane], L.d[j][1][1][lane]};
+                    n0 = mfma_split(p.k[0][1], d1, n0);
+                    n1 = mfma_split(p.k[1][1], d1, n1);
+                }
+                const float f = p.fk * fd[j];
+                st[j][0] = st[j][0] * p.gc + n0 * f;
+                st[j][1] = st[j][1] * p.gc + n1 * f;
+                publish(j);
+            }
+            lds_barrier();
+        };
+        GdnStateOps<NT> pa, pb;
+        load(pa, 0);
+#pragma unroll
+        for (int j = 0; j < NT; j++) publish(j);
+        lds_barrier();
+        for (uint32_t c = 0; c < nch; c += 2) {
+            load(pb, c + 1);
+            step(pa);
+            if (c + 1 == nch) break;
+            load(pa, c + 2);
+            step(pb);
+        }
+#pragma unroll
+        for (int j = 0; j < NT; j++)
+#pragma unroll
+            for (int t = 0; t < 2; t++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t i = 32 * w + 16 * t + 4 * g + r, col = j0 + 16 * j + m16;
+                    if (i < dk && col < dv) S[(size_t)i * dv + col] = st[j][t][r];
+                }
+    } else {
+        auto load = [&](GdnOutOps<NT> &p, uint32_t c) {
+            const char *b = scratch + (size_t)min(c, nch - 1) * CTOX_GDN_CHUNK_BYTES;
+            const uint4 *qp = (const uint4 *)(b + GF_Q) + 512 * w + lane, *ap = (const uint4 *)(b + GF_A) + 256 * w + lane;
+            const float *aux = (const float *)(b + GF_AUX);
+#pragma unroll
+            for (int k = 0; k < 4; k++)
+#pragma unroll
+                for (int x = 0; x < 2; x++) p.q[k][x] = qp[128 * k + 64 * x];
+            p.fq = *(const float4 *)(aux + 64 + 16 * w + 4 * g);
+#pragma unroll
+            for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
+            p.wn = aux[322];
+#pragma unroll
+            for (int u = 0; u < 2; u++)
+#pragma unroll
+                for (int x = 0; x < 2; x++) p.am[u][x] = ap[128 * u + 64 * x];
+            p.fa = *(const float4 *)(aux + 128 + 16 * w + 4 * g);
+        };
+        const size_t rowv = (size_t)a.heads * dv;
+        auto step = [&](const GdnOutOps<NT> &p, uint32_t c) {
+            gv4f o[NT];
+            float fd[NT];
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const float sf[4] = {L.sf[j][0][m16], L.sf[j][1][m16], L.sf[j][2][m16], L.sf[j][3][m16]};
+                o[j] = times_state<NT>(p.q, L, j, lane, sf);
+                fd[j] = pow2(d_exponent(p.mu[j], p.wn, sf) - 15);
+            }
+            lds_barrier();
+            const uint32_t t0 = (a.chunk0 + c) * a.chunk, n = min(a.chunk, a.tokens - t0);
+            float *out = a.out + (size_t)t0 * rowv + (size_t)h * dv + j0 + m16;
+#pragma unroll
+            for (int j = 0; j < NT; j++) {
+                const uint4 d0[2] = {L.d[j][0][0][lane], L.d[j][0][1][lane]};
+                gv4f x = mfma_split(p.am[0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+                if (w >= 2 && second) {  // strips 0 and 1 see no token of the second step
+                    const uint4 d1[2] = {L.d[j][1][0][lane], L.d[j][1][1][lane]};
+                    x = mfma_split(p.am[1], d1, x);
+                }
+                const float fq[4] = {p.fq.x, p.fq.y, p.fq.z, p.fq.w}, fa[4] = {p.fa.x, p.fa.y, p.fa.z, p.fa.w};
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const uint32_t s = 16 * w + 4 * g + r;
+                    if (s < n && j0 + 16 * j + m16 < dv) out[(size_t)s * rowv + 16 * j] = fq[r] * o[j][r] + fa[r] * fd[j] * x[r];
+                }
+            }
+            lds_barrier();
+        };
+        GdnOutOps<NT> pa, pb;
+        load(pa, 0);
+        lds_barrier();
+        for (uint32_t c = 0; c < nch; c += 2) {
+            load(pb, c + 1);
+            step(pa, c);
+            if (c + 1 == nch) break;
+            load(pa, c + 2);
+            step(pb, c + 1);
+        }
+    }
+}
+
+// _vec: key_dim, value_dim and the token strides are multiples of 4 and q, k, v 16-byte aligned.
+extern "C" __global__ __launch_bounds__(256, 3) void ctox_gdn_chunk_prep_gfx950(GdnArgs a) { chunk_prep<false>(a); }
+extern "C" __global__ __launch_bounds__(256, 3) void ctox_gdn_chunk_prep_vec_gfx950(GdnArgs a) { chunk_prep<true>(a); }
+extern "C" __global__ __launch_bounds__(512) void ctox_gdn_chunk_scan1_gfx950(GdnArgs a) { chunk_scan<1>(a); }
+extern "C" __global__ __launch_bounds__(512) void ctox_gdn_chunk_scan2_gfx950(GdnArgs a) { chunk_scan<2>(a); }

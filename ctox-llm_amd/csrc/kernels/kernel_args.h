@@ -241,6 +241,10 @@ struct RowDotArgs {
     uint32_t pad;
 };
 
+// Chunked prefill: scratch of one (head, chunk), the operands the sequential
+// pass reads (gated_delta_chunk.hip).
+#define CTOX_GDN_CHUNK_BYTES 148992
+
 // Gated-delta recurrence. State [heads][key_dim][value_dim] f32.
 struct GdnArgs {
     const float *q;         // [tokens][heads][key_dim]
@@ -250,7 +254,7 @@ struct GdnArgs {
     const float *beta;      // [tokens][heads]
     float *state;
     float *out;             // [tokens][heads][value_dim]
-    float *norms;           // chunked prefill scratch: per (head, chunk) T, A, G, k_inv, q_inv
+    float *norms;           // chunked prefill scratch: [head][chunk of the launch] CTOX_GDN_CHUNK_BYTES
     uint32_t tokens;
     uint32_t heads;
     uint32_t key_dim;
@@ -259,6 +263,8 @@ struct GdnArgs {
     uint32_t rep;           // value heads per key head: q, k of head h are key head h / rep
     uint32_t qk_stride;     // floats between tokens of q and of k
     uint32_t v_stride;      // floats between tokens of v
+    uint32_t chunk0;        // chunked prefill: the launch covers chunks chunk0 .. chunk0 + chunks - 1
+    uint32_t chunks;
     uint32_t pad;
 };
 

@@ -145,7 +145,7 @@ struct ctox_hip_backend {
     hipStream_t stream = nullptr;
     hipFunction_t prep = nullptr, q4_b1 = nullptr, q4_b4 = nullptr, q4_b8 = nullptr, q2_b1 = nullptr,
                   q2_b4 = nullptr, q2_b8 = nullptr, rec_row = nullptr, row_dot = nullptr,
-                  gdn_scan = nullptr, gdn_chunk_prep = nullptr, gdn_chunk_scan = nullptr, gdn_chunk_scan_vec = nullptr, gates = nullptr,
+                  gdn_scan = nullptr, gdn_chunk_prep[2] = {}, gdn_chunk_scan[2] = {}, gates = nullptr,
                   repeat = nullptr, partials = nullptr, argmax_final = nullptr, greedy_status = nullptr, verify = nullptr, decide = nullptr,
                   pick_sums = nullptr, pick_final = nullptr, rms = nullptr, swiglu = nullptr, sgate = nullptr,
                   conv = nullptr, rope = nullptr, kv_pack = nullptr, attn_prep = nullptr, kv_demote = nullptr, gqa_part[2] = {}, gqa_part16[2] = {},
@@ -888,9 +888,10 @@ extern "C" ctox_status ctox_hip_backend_create(int device, ctox_hip_backend **ou
                {&b->q4_b8, "ctox_q4_matvec_b8_gfx950"},    {&b->q2_b4, "ctox_q2_matvec_b4_gfx950"},
                {&b->q2_b8, "ctox_q2_matvec_b8_gfx950"},    {&b->rec_row, "ctox_recovered_row_gfx950"},
                {&b->row_dot, "ctox_row_dot_gfx950"},
-               {&b->gdn_scan, "ctox_gdn_scan_gfx950"},    {&b->gdn_chunk_prep, "ctox_gdn_chunk_prep_gfx950"},
-               {&b->gdn_chunk_scan, "ctox_gdn_chunk_scan_gfx950"},
-               {&b->gdn_chunk_scan_vec, "ctox_gdn_chunk_scan_vec_gfx950"}, {&b->gates, "ctox_gdn_gates_gfx950"},
+               {&b->gdn_scan, "ctox_gdn_scan_gfx950"},    {&b->gdn_chunk_prep[0], "ctox_gdn_chunk_prep_gfx950"},
+               {&b->gdn_chunk_prep[1], "ctox_gdn_chunk_prep_vec_gfx950"},
+               {&b->gdn_chunk_scan[0], "ctox_gdn_chunk_scan1_gfx950"},
+               {&b->gdn_chunk_scan[1], "ctox_gdn_chunk_scan2_gfx950"}, {&b->gates, "ctox_gdn_gates_gfx950"},
                {&b->repeat, "ctox_repeat_heads_gfx950"},   {&b->partials, "ctox_row_partials_gfx950"},
                {&b->argmax_final, "ctox_argmax_final_gfx950"}, {&b->greedy_status, "ctox_greedy_status_gfx950"}, {&b->verify, "ctox_verify_greedy_gfx950"},
                {&b->decide, "ctox_mtp_decide_gfx950"},     {&b->pick_sums, "ctox_pick_sums_gfx950"},
@@ -1710,6 +1711,9 @@ extern "C" ctox_status ctox_hip_recovered_row_matvec(ctox_hip_backend *b, const 
 // gated delta
 // ======================================================================
 namespace {
+// Scratch of a run of prefill chunks.
+constexpr size_t kGdnScratch = (size_t)160 << 20;
+
 ctox_status gdn_shape(size_t tokens, size_t heads, size_t kd, size_t vd) {
     if (tokens == 0 || heads == 0 || kd == 0 || vd == 0)
         return fail(CTOX_ERR_SHAPE, "delta shapes must be non-zero");
@@ -1738,8 +1742,11 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
     // 128 and chunks up to 64 tokens; otherwise the token-serial scan.
     const bool chunked = tokens > 1 && chunk >= 1 && chunk <= 64 && kd <= 128 && vd <= 128;
     const size_t nch = chunked ? (tokens + chunk - 1) / chunk : 0;
-    const size_t scratch = chunked ? heads * nch * (2 * 64 * 64 + 4 * 64) : 1;
-    st = ensure(b, b->norms, scratch * sizeof(float), false);
+    // The chunked passes alternate over runs of chunks, so that the scratch
+    // between them stays in the 256 MB Infinity Cache however long the prompt.
+    const size_t runs = (heads * nch * CTOX_GDN_CHUNK_BYTES + kGdnScratch - 1) / kGdnScratch;
+    const size_t run = chunked ? (nch + runs - 1) / runs : 0;
+    st = ensure(b, b->norms, chunked ? heads * run * CTOX_GDN_CHUNK_BYTES : sizeof(float), false);
     if (st) return st;
     GdnArgs a{};
     a.q = q;
@@ -1760,17 +1767,21 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
     a.v_stride = (uint32_t)v_stride;
     const size_t slices = (vd + 15) / 16;
     if (chunked) {
-        st = launch(b->gdn_chunk_prep, dim3((unsigned)(heads * nch)), dim3(256), s, a, "ctox_gdn_chunk_prep_gfx950");
-        if (st) return st;
-        // 8 * ceil(heads / 8) * slices workgroups: the kernel maps them so
-        // that all slices of a head run on one XCD (surplus ones exit).
-        // The vector instantiation: 16-byte branch-free loads; it needs the
-        // shapes, strides and alignment below.
-        const bool vec = kd % 4 == 0 && vd % 16 == 0 && qk_stride % 4 == 0 && v_stride % 4 == 0 &&
-                         (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0 && chunk * qk_stride < 0x1ffffff0u &&
-                         chunk * v_stride < 0x1ffffff0u;
-        return launch(vec ? b->gdn_chunk_scan_vec : b->gdn_chunk_scan, dim3((unsigned)(8 * ((heads + 7) / 8) * slices)),
-                      dim3(256), s, a, vec ? "ctox_gdn_chunk_scan_vec_gfx950" : "ctox_gdn_chunk_scan_gfx950");
+        // 16-byte reads of the q, k and v rows.
+        const int vec = kd % 4 == 0 && vd % 4 == 0 && qk_stride % 4 == 0 && v_stride % 4 == 0 &&
+                        (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
+        const unsigned heads8 = (unsigned)(8 * ((heads + 7) / 8));  // the kernels' XCD map; surplus workgroups exit
+        const int nt = heads * slices <= (size_t)b->cus ? 1 : 2;
+        for (size_t c0 = 0; c0 < nch; c0 += run) {
+            a.chunk0 = (uint32_t)c0;
+            a.chunks = (uint32_t)std::min(run, nch - c0);
+            st = launch(b->gdn_chunk_prep[vec], dim3(heads8 * a.chunks), dim3(256), s, a, "ctox_gdn_chunk_prep_gfx950");
+            if (!st)
+                st = launch(b->gdn_chunk_scan[nt - 1], dim3(heads8 * (unsigned)((vd + 16 * nt - 1) / (16 * nt))), dim3(512), s, a,
+                            "ctox_gdn_chunk_scan_gfx950");
+            if (st) return st;
+        }
+        return CTOX_OK;
     }
     return launch(b->gdn_scan, dim3((unsigned)(heads * slices)), dim3(256), s, a, "ctox_gdn_scan_gfx950");
 }
