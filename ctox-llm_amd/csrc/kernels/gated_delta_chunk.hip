@@ -505,13 +505,16 @@ struct GdnScanLds {
     float sf[NT][4][16];      // [value tile][key step][column]: what the state operand was divided by
 };
 
-// X = (rows) x S_0 with the key steps' column factors applied.
-template <int NT>
+// X = (rows) x S_0 with the key steps' column factors applied. fetch(k) issues
+// a quarter of the next chunk's loads.
+template <int NT, class Fetch>
 __device__ __forceinline__ gv4f times_state(const uint4 (&x)[4][2], const GdnScanLds<NT> &L, int j, uint32_t lane,
-                                            const float (&sf)[4]) {
+                                            const float (&sf)[4], Fetch fetch) {
     gv4f acc[4];
 #pragma unroll
     for (int k = 0; k < 4; k++) {
+        fetch(k);
+        __builtin_amdgcn_sched_barrier(0);
         const uint4 s[2] = {L.s[j][k][0][lane], L.s[j][k][1][lane]};
         acc[k] = mfma_split(x[k], s, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
     }
@@ -539,29 +542,34 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
     const bool second = a.chunk > 32;  // tokens in the second step
 
     if (wave < 4) {
-        auto load = [&](GdnStateOps<NT> &p, uint32_t c) {
+        // part 0..3: W of a key step (and the small operands), 4: K^T of the first key tile, 5: of the second.
+        auto load = [&](GdnStateOps<NT> &p, uint32_t c, int part) {
             const char *b = scratch + (size_t)min(c, nch - 1) * CTOX_GDN_CHUNK_BYTES;
             const uint4 *wp = (const uint4 *)(b + GF_W) + 512 * w + lane, *kp = (const uint4 *)(b + GF_K) + 512 * w + lane;
             const float4 *up = (const float4 *)(b + GF_U) + 256 * (NT * slice) + 64 * w + lane;
             const float *aux = (const float *)(b + GF_AUX);
+            if (part < 4) {
 #pragma unroll
-            for (int k = 0; k < 4; k++)
+                for (int x = 0; x < 2; x++) p.w[part][x] = wp[128 * part + 64 * x];
+            }
+            if (part == 0) {
 #pragma unroll
-                for (int x = 0; x < 2; x++) p.w[k][x] = wp[128 * k + 64 * x];
+                for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
+                p.wn = aux[322];
+                p.gc = aux[320];
+                p.fk = aux[321];
+            }
+            if (part == 1) {
 #pragma unroll
-            for (int j = 0; j < NT; j++) p.u[j] = up[256 * j];
-            p.fw = *(const float4 *)(aux + 16 * w + 4 * g);
-#pragma unroll
-            for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
-            p.wn = aux[322];
-#pragma unroll
-            for (int t = 0; t < 2; t++)
+                for (int j = 0; j < NT; j++) p.u[j] = up[256 * j];
+                p.fw = *(const float4 *)(aux + 16 * w + 4 * g);
+            }
+            if (part >= 4) {
 #pragma unroll
                 for (int u = 0; u < 2; u++)
 #pragma unroll
-                    for (int x = 0; x < 2; x++) p.k[t][u][x] = kp[256 * t + 128 * u + 64 * x];
-            p.gc = aux[320];
-            p.fk = aux[321];
+                    for (int x = 0; x < 2; x++) p.k[part - 4][u][x] = kp[256 * (part - 4) + 128 * u + 64 * x];
+            }
         };
         // State rows 32 w + 16 t + 4 g + r, column j0 + 16 j + m16.
         gv4f st[NT][2];
@@ -591,12 +599,14 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
             L.s[j][w][1][lane] = f[1];
             if (g == 0) L.sf[j][w][m16] = pow2(e - 15);
         };
-        auto step = [&](const GdnStateOps<NT> &p) {
+        auto step = [&](const GdnStateOps<NT> &p, GdnStateOps<NT> &nx, uint32_t c) {
             float fd[NT];
 #pragma unroll
             for (int j = 0; j < NT; j++) {
                 const float sf[4] = {L.sf[j][0][m16], L.sf[j][1][m16], L.sf[j][2][m16], L.sf[j][3][m16]};
-                const gv4f x = times_state<NT>(p.w, L, j, lane, sf);
+                const gv4f x = times_state<NT>(p.w, L, j, lane, sf, [&](int k) {
+                    if (j == 0) load(nx, c + 1, k);
+                });
                 const int e = d_exponent(p.mu[j], p.wn, sf);
                 const float sc = pow2(15 - e);
                 fd[j] = pow2(e - 15);
@@ -609,6 +619,7 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < NT; j++) {
+                if (j == 0) load(nx, c + 1, 4);
                 const uint4 d0[2] = {L.d[j][0][0][lane], L.d[j][0][1][lane]};
                 gv4f n0 = mfma_split(p.k[0][0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
                 gv4f n1 = mfma_split(p.k[1][0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
@@ -617,6 +628,8 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
                     n0 = mfma_split(p.k[0][1], d1, n0);
                     n1 = mfma_split(p.k[1][1], d1, n1);
                 }
+                __builtin_amdgcn_sched_barrier(0);
+                if (j == 0) load(nx, c + 1, 5);
                 const float f = p.fk * fd[j];
                 st[j][0] = st[j][0] * p.gc + n0 * f;
                 st[j][1] = st[j][1] * p.gc + n1 * f;
@@ -625,16 +638,15 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
             lds_barrier();
         };
         GdnStateOps<NT> pa, pb;
-        load(pa, 0);
+#pragma unroll
+        for (int part = 0; part < 6; part++) load(pa, 0, part);
 #pragma unroll
         for (int j = 0; j < NT; j++) publish(j);
         lds_barrier();
         for (uint32_t c = 0; c < nch; c += 2) {
-            load(pb, c + 1);
-            step(pa);
+            step(pa, pb, c);
             if (c + 1 == nch) break;
-            load(pa, c + 2);
-            step(pb);
+            step(pb, pa, c + 1);
         }
 #pragma unroll
         for (int j = 0; j < NT; j++)
@@ -646,35 +658,44 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
                     if (i < dk && col < dv) S[(size_t)i * dv + col] = st[j][t][r];
                 }
     } else {
-        auto load = [&](GdnOutOps<NT> &p, uint32_t c) {
+        // part 0..3: Q of a key step (and the small operands), 4, 5: A of a token step.
+        auto load = [&](GdnOutOps<NT> &p, uint32_t c, int part) {
             const char *b = scratch + (size_t)min(c, nch - 1) * CTOX_GDN_CHUNK_BYTES;
             const uint4 *qp = (const uint4 *)(b + GF_Q) + 512 * w + lane, *ap = (const uint4 *)(b + GF_A) + 256 * w + lane;
             const float *aux = (const float *)(b + GF_AUX);
+            if (part < 4) {
 #pragma unroll
-            for (int k = 0; k < 4; k++)
+                for (int x = 0; x < 2; x++) p.q[part][x] = qp[128 * part + 64 * x];
+            }
+            if (part == 0) {
 #pragma unroll
-                for (int x = 0; x < 2; x++) p.q[k][x] = qp[128 * k + 64 * x];
-            p.fq = *(const float4 *)(aux + 64 + 16 * w + 4 * g);
+                for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
+                p.wn = aux[322];
+            }
+            if (part == 1) {
+                p.fq = *(const float4 *)(aux + 64 + 16 * w + 4 * g);
+                p.fa = *(const float4 *)(aux + 128 + 16 * w + 4 * g);
+            }
+            if (part >= 4) {
 #pragma unroll
-            for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
-            p.wn = aux[322];
-#pragma unroll
-            for (int u = 0; u < 2; u++)
-#pragma unroll
-                for (int x = 0; x < 2; x++) p.am[u][x] = ap[128 * u + 64 * x];
-            p.fa = *(const float4 *)(aux + 128 + 16 * w + 4 * g);
+                for (int x = 0; x < 2; x++) p.am[part - 4][x] = ap[128 * (part - 4) + 64 * x];
+            }
         };
         const size_t rowv = (size_t)a.heads * dv;
-        auto step = [&](const GdnOutOps<NT> &p, uint32_t c) {
+        auto step = [&](const GdnOutOps<NT> &p, GdnOutOps<NT> &nx, uint32_t c) {
             gv4f o[NT];
             float fd[NT];
 #pragma unroll
             for (int j = 0; j < NT; j++) {
                 const float sf[4] = {L.sf[j][0][m16], L.sf[j][1][m16], L.sf[j][2][m16], L.sf[j][3][m16]};
-                o[j] = times_state<NT>(p.q, L, j, lane, sf);
+                o[j] = times_state<NT>(p.q, L, j, lane, sf, [&](int k) {
+                    if (j == 0) load(nx, c + 1, k);
+                });
                 fd[j] = pow2(d_exponent(p.mu[j], p.wn, sf) - 15);
             }
             lds_barrier();
+            load(nx, c + 1, 4);
+            load(nx, c + 1, 5);
             const uint32_t t0 = (a.chunk0 + c) * a.chunk, n = min(a.chunk, a.tokens - t0);
             float *out = a.out + (size_t)t0 * rowv + (size_t)h * dv + j0 + m16;
 #pragma unroll
@@ -695,14 +716,13 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
             lds_barrier();
         };
         GdnOutOps<NT> pa, pb;
-        load(pa, 0);
+#pragma unroll
+        for (int part = 0; part < 6; part++) load(pa, 0, part);
         lds_barrier();
         for (uint32_t c = 0; c < nch; c += 2) {
-            load(pb, c + 1);
-            step(pa, c);
+            step(pa, pb, c);
             if (c + 1 == nch) break;
-            load(pa, c + 2);
-            step(pb, c + 1);
+            step(pb, pa, c + 1);
         }
     }
 }
