@@ -1711,7 +1711,10 @@ extern "C" ctox_status ctox_hip_recovered_row_matvec(ctox_hip_backend *b, const 
 // gated delta
 // ======================================================================
 namespace {
-// Scratch of a run of prefill chunks.
+// Scratch of a run of prefill chunks: runs short enough that the sequential
+// pass finds their operands in the 256 MB Infinity Cache, long enough that the
+// launches fill the CUs (4096 tokens of 32 heads, 305 MB in all: 400 us at 48 MB,
+// 266 at 96, 245 at 160, 318 in one run).
 constexpr size_t kGdnScratch = (size_t)160 << 20;
 
 ctox_status gdn_shape(size_t tokens, size_t heads, size_t kd, size_t vd) {
@@ -1742,8 +1745,7 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
     // 128 and chunks up to 64 tokens; otherwise the token-serial scan.
     const bool chunked = tokens > 1 && chunk >= 1 && chunk <= 64 && kd <= 128 && vd <= 128;
     const size_t nch = chunked ? (tokens + chunk - 1) / chunk : 0;
-    // The chunked passes alternate over runs of chunks, so that the scratch
-    // between them stays in the 256 MB Infinity Cache however long the prompt.
+    // The chunked passes alternate over runs of chunks (kGdnScratch).
     const size_t runs = (heads * nch * CTOX_GDN_CHUNK_BYTES + kGdnScratch - 1) / kGdnScratch;
     const size_t run = chunked ? (nch + runs - 1) / runs : 0;
     st = ensure(b, b->norms, chunked ? heads * run * CTOX_GDN_CHUNK_BYTES : sizeof(float), false);
@@ -1771,11 +1773,13 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
         const int vec = kd % 4 == 0 && vd % 4 == 0 && qk_stride % 4 == 0 && v_stride % 4 == 0 &&
                         (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
         const unsigned heads8 = (unsigned)(8 * ((heads + 7) / 8));  // the kernels' XCD map; surplus workgroups exit
+        // 16-column slices while every (head, slice) has a CU of its own (35 us per 20 chunks of 32 heads,
+        // 47 with 32 columns); else 32, whose products share the loaded operands.
         const int nt = heads * slices <= (size_t)b->cus ? 1 : 2;
         for (size_t c0 = 0; c0 < nch; c0 += run) {
             a.chunk0 = (uint32_t)c0;
             a.chunks = (uint32_t)std::min(run, nch - c0);
-            st = launch(b->gdn_chunk_prep[vec], dim3(heads8 * a.chunks), dim3(256), s, a, "ctox_gdn_chunk_prep_gfx950");
+            st = launch(b->gdn_chunk_prep[vec], dim3((unsigned)heads * a.chunks), dim3(256), s, a, "ctox_gdn_chunk_prep_gfx950");
             if (!st)
                 st = launch(b->gdn_chunk_scan[nt - 1], dim3(heads8 * (unsigned)((vd + 16 * nt - 1) / (16 * nt))), dim3(512), s, a,
                             "ctox_gdn_chunk_scan_gfx950");

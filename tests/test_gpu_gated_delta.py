@@ -102,6 +102,29 @@ def test_chunked_prefill_ragged(hip, orc, case):
     close(st_gpu, st_ref, 1e-4, "state")
 
 
+@pytest.mark.parametrize("heads,dv,vs,ss,bmax,ldmax", [
+    (2, 128, 1e6, 1e-3, 1.0, 0.0), (40, 48, 1e-6, 1e5, 1.0, 0.0), (3, 100, 1e30, 1.0, 1.0, 0.0),
+    (40, 128, 1e-30, 1e-25, 1.0, 0.0), (2, 16, 1.0, 1.0, 2.0, 0.02), (1, 128, 0.0, 0.0, 1.0, 0.0)])
+def test_chunked_prefill_magnitudes(hip, orc, heads, dv, vs, ss, bmax, ldmax):
+    """The chunked path's operands are split into f16 parts after scaling by
+    powers of two: values and states of any fp32 magnitude (mixed ones too),
+    beta up to 2, decays above one and an all-zero run give what the oracle
+    gives. 40 heads of 48 / 128 columns take the two-tile slices, fewer the
+    one-tile ones. Tolerances as above, relative to the reference's rms."""
+    T, dk, chunk = 200, 128, 64
+    say(f"case gdn magnitudes heads={heads} dv={dv} v={vs} s={ss}")
+    q, k, v, ld, be = gdn_inputs(T, heads, heads, dk, dv, heads + dv)
+    v, be, ld = (v * np.float32(vs)).astype(np.float32), (be * np.float32(bmax)).astype(np.float32), ld
+    if ldmax:
+        ld = np.random.default_rng(1).uniform(-0.05, ldmax, ld.shape).astype(np.float32)
+    st_ref = (np.random.default_rng(T).standard_normal(heads * dk * dv) * ss).astype(np.float32)
+    st_gpu = st_ref.copy()
+    ref = orc.gated_delta_sequence(q, k, v, ld, be, st_ref, T, heads, dk, dv)
+    got = hip.gated_delta_sequence(q, k, v, ld, be, st_gpu, T, heads, dk, dv, chunk)
+    close(got, ref, 1e-3, "output")
+    close(st_gpu, st_ref, 1e-4, "state")
+
+
 @pytest.mark.parametrize("T", [1024, 4096])
 def test_chunked_prefill_long(hip, orc, T):
     """BASELINE config 4 shapes through the chunk-64 path, up to the config's
