@@ -119,6 +119,10 @@ __device__ __forceinline__ int exponent_of(float x) {
 }
 __device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
 
+// exp(x) whose relative error grows with |x| (2^-24 |x|): for decay factors,
+// where |x| exp(x) <= 1/e keeps it under 2^-25 of one.
+__device__ __forceinline__ float exp_decay(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
+
 // Sum / max over the four lane groups (lanes l, l ^ 16, l ^ 32).
 __device__ __forceinline__ float groups_sum(float v) {
     v += __shfl_xor(v, 16);
@@ -186,7 +190,7 @@ template <bool VEC>
 __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     __shared__ __align__(16) float kh[GC * SPAD];  // raw K rows, then V rows
     __shared__ float tt[GC * TPAD];                // L, T0, W's and then U's left operand
-    __shared__ float G[GC], bt[GC], kinv_s[GC], ekf[GC];
+    __shared__ __align__(16) float G[GC], bt[GC], kinv_s[GC], ekf[GC];
     __shared__ float wsq[4][GC];
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t m16 = lane & 15, g = lane >> 4;
@@ -281,13 +285,15 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     }
     {   // A: row t = own, this lane's r = 16 u + 4 g + x
         float sq = 0.0f;
+        const float Gown = G[own];
 #pragma unroll
         for (uint32_t u = 0; u < 4; u++) {
             if (u > w) continue;
+            const gv4f Gr = *(const gv4f *)&G[16 * u + 4 * g], kr4 = *(const gv4f *)&kinv_s[16 * u + 4 * g];
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 const uint32_t r = 16 * u + 4 * g + x;
-                const float val = r <= own ? expf(G[own] - G[r]) * (kinv_s[r] * qinv) * acc[u][x] : 0.0f;
+                const float val = r <= own ? exp_decay(Gown - Gr[x]) * (kr4[x] * qinv) * acc[u][x] : 0.0f;
                 acc[u][x] = val;
                 sq += val * val;
             }
@@ -311,10 +317,11 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
 #pragma unroll
         for (uint32_t u = 1; u < 5; u++) {
             if (u <= w) continue;
+            const gv4f kr4 = *(const gv4f *)&kinv_s[16 * (u - w - 1) + 4 * g];
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 const uint32_t r = 16 * (u - w - 1) + 4 * g + x;
-                tt[s * TPAD + r] = r < s ? f * kinv_s[r] * acc[u][x] : 0.0f;
+                tt[s * TPAD + r] = r < s ? f * kr4[x] * acc[u][x] : 0.0f;
             }
         }
     }
@@ -344,12 +351,12 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
             const float *kp = kh + 16 * (2 * w + t) + m16;
 #pragma unroll
             for (int st = 0; st < 2; st++) {
-                gv4f lo, up;
+                gv4f lo = *(const gv4f *)&ekf[32 * st + 4 * g], up = *(const gv4f *)&ekf[32 * st + 16 + 4 * g];
 #pragma unroll
                 for (int x = 0; x < 4; x++) {
                     const uint32_t r = 32 * st + 4 * g + x;
-                    lo[x] = kp[r * SPAD] * ekf[r];
-                    up[x] = kp[(r + 16) * SPAD] * ekf[r + 16];
+                    lo[x] *= kp[r * SPAD];
+                    up[x] *= kp[(r + 16) * SPAD];
                 }
                 uint4 f[2];
                 split8(lo, up, f);
@@ -394,7 +401,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         for (int i = 0; i < 16; i++) {
             const uint32_t s = 16 * w + i;
             const float t = tt[s * TPAD + lane] * b;
-            tu[i] = lane <= s ? t * expf(G[s] - gl) : 0.0f;
+            tu[i] = lane <= s ? t * exp_decay(G[s] - gl) : 0.0f;
             tt[s * TPAD + lane] = t * ki;
         }
     }

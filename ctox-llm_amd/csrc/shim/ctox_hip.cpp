@@ -148,7 +148,7 @@ struct ctox_hip_backend {
                   gdn_scan = nullptr, gdn_chunk_prep[2] = {}, gdn_chunk_scan[2] = {}, gates = nullptr,
                   repeat = nullptr, partials = nullptr, argmax_final = nullptr, greedy_status = nullptr, verify = nullptr, decide = nullptr,
                   pick_sums = nullptr, pick_final = nullptr, rms = nullptr, swiglu = nullptr, sgate = nullptr,
-                  conv = nullptr, rope = nullptr, kv_pack = nullptr, attn_prep = nullptr, kv_demote = nullptr, gqa_part[2] = {}, gqa_part16[2] = {},
+                  conv = nullptr, rope = nullptr, kv_pack = nullptr, attn_prep = nullptr, kv_demote = nullptr, gqa_part[2] = {}, gqa_tiles[2] = {},
                   gqa_combine = nullptr, fill = nullptr, embed = nullptr, norm_rows = nullptr, attn_gate = nullptr,
                   swiglu_rows = nullptr, copy_rows = nullptr, write_words = nullptr, norm_prep = nullptr,
                   prep_x = nullptr, finite = nullptr, gather = nullptr, topk_part = nullptr, topk_final = nullptr, stream_read = nullptr,
@@ -901,8 +901,8 @@ extern "C" ctox_status ctox_hip_backend_create(int device, ctox_hip_backend **ou
                {&b->kv_pack, "ctox_kv_pack_q4_gfx950"}, {&b->attn_prep, "ctox_attn_prep_gfx950"},    {&b->kv_demote, "ctox_kv_demote_gfx950"},
                {&b->gqa_part[0], "ctox_paged_gqa_partial_r1_gfx950"},
                {&b->gqa_part[1], "ctox_paged_gqa_partial_r2_gfx950"},
-               {&b->gqa_part16[0], "ctox_paged_gqa_partial16_r1_gfx950"},
-               {&b->gqa_part16[1], "ctox_paged_gqa_partial16_r2_gfx950"},
+               {&b->gqa_tiles[0], "ctox_paged_gqa_tiles_r1_gfx950"},
+               {&b->gqa_tiles[1], "ctox_paged_gqa_tiles_r2_gfx950"},
                {&b->gqa_combine, "ctox_paged_gqa_combine_gfx950"},
                {&b->fill, "ctox_fill_random_gfx950"},      {&b->embed, "ctox_embed_rows_gfx950"},
                {&b->norm_rows, "ctox_norm_rows_gfx950"},   {&b->attn_gate, "ctox_attn_gate_gfx950"},
@@ -2398,12 +2398,16 @@ ctox_status paged_gqa_impl(ctox_hip_backend *b, const float *d_query, const uint
         return fail(CTOX_ERR_SHAPE, "paged KV geometry differs from the attention contract");
     const uint32_t queries = group * (uint32_t)rows;
     const uint32_t tiles = (p->tokens + 15) / 16;
-    // Two workgroups per CU for the 16-query kernel (it fits two per CU), one for the 32-query one.
-    const uint32_t per_cu = queries > 16 ? 1 : 2;
+    // Page-aligned 16-token tiles take the int8-MFMA kernel (a workgroup walks steps of 16 tiles), other
+    // page sizes the fp32-MFMA one (its four waves take a run of tiles each). Two workgroups per CU for up
+    // to 16 queries, one for up to 32 (the registers and LDS they fit).
+    const bool aligned = p->page_tokens % 16 == 0;
+    const uint32_t per_cu = queries > 16 ? 1 : 2, unit = aligned ? 16 : 4;
     uint32_t splits = std::max<uint32_t>(1, (uint32_t)((per_cu * b->cus + p->key_value_heads - 1) / p->key_value_heads));
-    splits = std::min<uint32_t>(std::min<uint32_t>(splits, (tiles + 3) / 4), 1024);
-    const uint32_t tpw = (tiles + 4 * splits - 1) / (4 * splits);
-    splits = (tiles + 4 * tpw - 1) / (4 * tpw);
+    splits = std::min<uint32_t>(std::min<uint32_t>(splits, (tiles + unit - 1) / unit), 1024);
+    const uint32_t per_wg = (tiles + unit * splits - 1) / (unit * splits) * unit;  // tiles
+    splits = (tiles + per_wg - 1) / per_wg;
+    const uint32_t tpw = aligned ? per_wg : per_wg / 4;
     const size_t part = (size_t)p->key_value_heads * splits * queries;
     ctox_status st = ensure(b, b->attn, part * (256 + 2) * sizeof(float), false);
     if (st) return st;
@@ -2411,7 +2415,7 @@ ctox_status paged_gqa_impl(ctox_hip_backend *b, const float *d_query, const uint
     GqaArgs a{d_query, d_q2_pages, d_q4_pages, (const PagedKvDesc *)d_descriptors, part_out, part_out + part * 256,
               d_out, p->q2_page_bytes, p->q4_page_bytes, p->query_heads, group, p->tokens, (uint32_t)rows, queries,
               p->page_tokens, p->page_count, (uint32_t)cv, p->q2_token_bytes, p->q4_token_bytes, tiles, tpw, splits,
-              p->scale, p->page_tokens % 16 == 0 ? 1u : 0u, 0};
+              p->scale, aligned ? 1u : 0u, 0};
     if (gs) {
         const int layout = gs->dtype == CTOX_DTYPE_Q4B64 ? 1 : 0;
         const size_t blocks = (size_t)p->query_heads * 256 / kBlockLen;
@@ -2426,11 +2430,8 @@ ctox_status paged_gqa_impl(ctox_hip_backend *b, const float *d_query, const uint
         a.st_dtype = (uint32_t)layout;
     }
     hipStream_t s = pick_stream(b, stream);
-    // Page-aligned 16-token tiles run P.V on f16 MFMA; other page sizes on the fp32-MFMA kernel.
-    // (its waves hold up to 64 tiles' page descriptors in registers).
-    const bool f16 = p->page_tokens % 16 == 0 && tpw <= 64;
-    hipFunction_t part_fn = f16 ? b->gqa_part16[queries > 16 ? 1 : 0] : b->gqa_part[queries > 16 ? 1 : 0];
-    st = launch(part_fn, dim3(splits, p->key_value_heads), dim3(256), s, a,
+    hipFunction_t part_fn = aligned ? b->gqa_tiles[queries > 16 ? 1 : 0] : b->gqa_part[queries > 16 ? 1 : 0];
+    st = launch(part_fn, dim3(splits, p->key_value_heads), dim3(aligned && queries > 16 ? 512 : 256), s, a,
                 "ctox_paged_gqa_partial_gfx950");
     if (st) return st;
     return launch(b->gqa_combine, dim3(queries, p->key_value_heads, 4), dim3(256), s, a, "ctox_paged_gqa_combine_gfx950");
