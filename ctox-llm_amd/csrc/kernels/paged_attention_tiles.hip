@@ -7,10 +7,15 @@
 // scores tokens 64 w .. 64 w + 63 of a step (four 16-token tiles), and then
 // owns value dims 64 w .. 64 w + 63 for all of the step's tokens.
 //
-//  Scores S = K Q^T, per 64-dim block: lane (li, lg) reads token li's block lg
-//  whole (16 B of Q2 codes or 32 B of Q4, straight from the page); a 4 x 4 lane
-//  transpose leaves it quarter lg of every block, which is its A operand, as
-//  bytes 2 code. The query is a fixed point X of 22 bits per query row, in three
+//  A token's K (V) head run is four blocks, 72 bytes Q2 or 136 Q4: consecutive
+//  lanes read its consecutive 8 bytes, and an LDS pass hands lane (li, lg) block
+//  lg of token li, scale and codes. (Each lane reading its own block's 16 bytes,
+//  18 or 34 apart and 2 off alignment, took about 60 cycles per load: 3.6 us of a
+//  256-token step.)
+//
+//  Scores S = K Q^T, per 64-dim block: a 4 x 4 lane transpose leaves a lane
+//  quarter lg of each of its token's blocks, which is its A operand, as bytes
+//  2 code. The query is a fixed point X of 22 bits per query row, in three
 //  balanced int8 limbs, and sum X (2 code - K) (K = 3 Q2, 15 Q4) is formed in
 //  int32 exactly: the -K sum X enters as the MFMA's C operand. One conversion
 //  and one fma with the block's scale per (token, query, block).
@@ -33,19 +38,16 @@
 // f16-MFMA kernel before took 750 per 16-token tile, 3000 for the same tokens).
 
 typedef int pt_v2i __attribute__((ext_vector_type(2)));
-struct __attribute__((packed, aligned(2))) PtCodes {  // 16 bytes of codes: they follow a 2-byte scale
-    uint32_t x[4];
-};
-
 #define PT_STEP 256   // tokens per step
-#define PT_RS2 72     // LDS bytes of one token's V codes (4 blocks): Q2 (64 + 8: the transposed reads of
-#define PT_RS4 136    // 64 tokens spread over the banks), Q4
+#define PT_RS 136     // LDS bytes of one token's V codes (4 blocks of 32, or 16; + 8: the transposed reads of 64
+                      // tokens spread over the banks)
 
 template <int R>
 struct PtLds {
     int8_t limbs[3][16 * R][PA_QB];
-    uint8_t v[PT_STEP * PT_RS4];
-    float p[R][4][4][64][4];         // [query tile][64-token part][token tile][lane][token 4 lg + c]
+    uint8_t v[PT_STEP * PT_RS];
+    float p[R][4][4][64][4];         // [query tile][64-token part][token tile][lane][token 4 lg + c]; before
+                                     // that a wave's part stages its keys
     float ksc[4 * R][4][4][16];      // [wave][tile][block][token]: K scale / K
     float vsc[4][PT_STEP];           // [block][token]: V scale
     float smax[4][R][16];
@@ -67,6 +69,14 @@ __device__ __forceinline__ void pt_limbs4(uint32_t z0, uint32_t z1, uint32_t z2,
     l2 = (u01 | u23) ^ 0x80808080u;
 }
 
+// Over a row of 16 lanes (DPP rotations, no LDS trip).
+__device__ __forceinline__ uint32_t pt_row_umax(uint32_t v) {
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x128, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x124, 0xF, 0xF, false));
+    v = max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x122, 0xF, 0xF, false));
+    return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, 0x121, 0xF, 0xF, false));
+}
+
 // Queries to limbs: thread i takes (query, block, quarter) = (i / 16, i / 4 % 4,
 // i % 4). X = rint(q 2^E), |X| <= 2^21, E from the query row's largest |q|. A
 // quarter's 16 dims are stored as byte 4 j + i of dim 4 i + j, the order in which
@@ -77,8 +87,7 @@ __device__ __forceinline__ void pt_prep(const GqaArgs &a, const float (&q)[16], 
     float mx = 0.0f;
 #pragma unroll
     for (int d = 0; d < 16; d++) mx = fmaxf(mx, fabsf(q[d]));
-#pragma unroll
-    for (int o = 1; o < 16; o <<= 1) mx = fmaxf(mx, __shfl_xor(mx, o));
+    mx = __uint_as_float(pt_row_umax(__float_as_uint(mx)));  // (magnitudes order as their bits)
     int ex = 0;
     frexpf(mx, &ex);  // mx < 2^ex
     const float e = mx > 0.0f ? ldexpf(1.0f, 21 - ex) : 0.0f;
@@ -96,19 +105,68 @@ __device__ __forceinline__ void pt_prep(const GqaArgs &a, const float (&q)[16], 
 #pragma unroll
     for (int k = 0; k < 3; k++)
         *(uint4 *)&L.limbs[k][qi][64 * b + 16 * part] = make_uint4(l[k][0], l[k][1], l[k][2], l[k][3]);
-    sum += __shfl_xor(sum, 1);
-    sum += __shfl_xor(sum, 2);
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, false);  // the quad's lanes
+    sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xF, 0xF, false);
     if (part == 0) L.xs[qi][b] = sum;
     if (b == 0 && part == 0) L.qs[qi] = mx > 0.0f ? ldexpf(a.scale * PA_LOG2E, ex - 21) : 0.0f;
 }
 
-// One wave's four tiles of a step in registers.
+// Where a wave's four tiles of a step lie (uniform).
 struct PtTiles {
-    PtCodes k[4][2], v[4][2];   // [tile][second half: Q4 only]
-    uint16_t ks[4], vs[4];      // fp16 scales of (token li, block lg)
-    uint32_t lo[4], hi[4];      // tokens [lo, hi) of the tile's page are held (uniform)
-    uint32_t q4;                // tiles in Q4 pages (uniform bits)
+    const uint8_t *page[4];
+    uint32_t lo[4], hi[4];  // tokens [lo, hi) are held
+    uint32_t q4;            // bit i: tile i lies in a Q4 page
 };
+
+// desc: lane at + i holds the page of the wave's tile i.
+__device__ __forceinline__ void pt_tiles(const GqaArgs &a, const uint4 &desc, uint32_t at, PtTiles &t) {
+    t.q4 = 0;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        const uint32_t prec = __builtin_amdgcn_readlane(desc.x, at + i), slot = __builtin_amdgcn_readlane(desc.y, at + i);
+        const uint32_t cnt = __builtin_amdgcn_readlane(desc.z, at + i), first = __builtin_amdgcn_readlane(desc.w, at + i);
+        t.q4 |= prec != 0 ? 1u << i : 0u;
+        t.lo[i] = first;
+        t.hi[i] = min(first + cnt, a.tokens);
+        t.page[i] = prec != 0 ? a.q4 + (size_t)slot * a.q4_page_bytes : a.q2 + (size_t)slot * a.q2_page_bytes;
+    }
+}
+
+// 8-byte pieces of a tile's 16 head runs: piece e = 64 n + lane is part e % P of token e / P, P = 9
+// (Q2) or 17 (Q4; of a Q2 page's tile there, 9 parts exist). Lanes without a piece or a token read
+// the query buffer, which is never used.
+template <int N, int P>
+__device__ __forceinline__ void pt_load(const GqaArgs &a, const uint8_t *page, uint32_t lo, uint32_t hi, uint32_t tb,
+                                        uint32_t run, uint32_t token_bytes, uint32_t parts, uint32_t lane, uint2 (&r)[N]) {
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        const uint32_t e = 64 * n + lane, tok = e / P, j = tb + tok;
+        const bool ok = e < 16 * P && e % P < parts && j >= lo && j < hi;
+        const uint8_t *p = ok ? page + (j - lo) * token_bytes + run + 8 * (e % P) : (const uint8_t *)a.query;
+        r[n] = make_uint2(((const uint32_t *)p)[0], ((const uint32_t *)p)[1]);
+    }
+}
+// The pieces to rows of PT_RS bytes, and block lg of row li back: its scale and 4 (8) words of codes.
+// Block lg starts at bs lg bytes (bs 18 or 34), i.e. its codes at a word or two bytes past one.
+template <int N, int P>
+__device__ __forceinline__ void pt_stage(uint8_t *rows, uint32_t bs, uint32_t lane, const uint2 (&r)[N],
+                                         uint32_t (&codes)[8], uint32_t &scale) {
+#pragma unroll
+    for (int n = 0; n < N; n++) {
+        const uint32_t e = 64 * n + lane;
+        if (e < 16 * P) *(uint2 *)(rows + e / P * PT_RS + 8 * (e % P)) = r[n];
+    }
+    constexpr int W = P == 9 ? 4 : 8;
+    const uint32_t start = (lane >> 4) * bs;
+    const uint8_t *row = rows + (lane & 15) * PT_RS;
+    scale = *(const uint16_t *)(row + start);
+    const uint32_t *w = (const uint32_t *)(row + ((start + 2) & ~3u));
+    uint32_t x[W + 1];
+#pragma unroll
+    for (int i = 0; i <= W; i++) x[i] = w[i];
+#pragma unroll
+    for (int i = 0; i < W; i++) codes[i] = __builtin_amdgcn_alignbyte(x[i + 1], x[i], (start + 2) & 3u);
+}
 
 // Q2 codes c as Q4 codes 5 c: (2 * 5 c - 15) / 15 = (2 c - 3) / 3, the same value.
 __device__ __forceinline__ uint32_t pt_widen8(uint32_t x) {  // 8 crumbs in the low half
@@ -117,76 +175,57 @@ __device__ __forceinline__ uint32_t pt_widen8(uint32_t x) {  // 8 crumbs in the 
     x = (x | (x << 2)) & 0x33333333u;
     return x | (x << 2);
 }
-__device__ __forceinline__ void pt_widen(PtCodes (&c)[2]) {
-    uint32_t w[8];
+__device__ __forceinline__ void pt_widen(uint32_t (&c)[8]) {
 #pragma unroll
-    for (int i = 0; i < 4; i++) {
-        w[2 * i] = pt_widen8(c[0].x[i] & 0xffffu);
-        w[2 * i + 1] = pt_widen8(c[0].x[i] >> 16);
+    for (int i = 3; i >= 0; i--) {
+        c[2 * i + 1] = pt_widen8(c[i] >> 16);
+        c[2 * i] = pt_widen8(c[i] & 0xffffu);
     }
-#pragma unroll
-    for (int i = 0; i < 8; i++) c[i / 4].x[i % 4] = w[i];
 }
 
-// Q4: 0 no tile of the workgroup lies in a Q4 page; 1 some do, and tiles of Q2 pages are widened.
-// desc: lane i < 4 holds the page of the wave's tile i. A lane without a token reads the query
-// buffer, which is never used.
-template <int Q4>
-__device__ __forceinline__ void pt_load(const GqaArgs &a, const uint4 &desc, uint32_t tb, uint32_t h, uint32_t li,
-                                        uint32_t lg, PtTiles &t) {
-    t.q4 = 0;
-#pragma unroll
-    for (int i = 0; i < 4; i++) {
-        const uint32_t prec = __builtin_amdgcn_readlane(desc.x, i), slot = __builtin_amdgcn_readlane(desc.y, i);
-        const uint32_t cnt = __builtin_amdgcn_readlane(desc.z, i), first = __builtin_amdgcn_readlane(desc.w, i);
-        const bool q4 = Q4 && prec != 0;
-        t.q4 |= q4 ? 1u << i : 0u;
-        t.lo[i] = first;
-        t.hi[i] = min(first + cnt, a.tokens);
-        const uint32_t bs = q4 ? 34u : 18u, j = tb + 16 * i + li;
-        const uint8_t *page = q4 ? a.q4 + (size_t)slot * a.q4_page_bytes : a.q2 + (size_t)slot * a.q2_page_bytes;
-        const bool ok = j >= t.lo[i] && j < t.hi[i];
-        const uint8_t *kp = ok ? page + (j - first) * (q4 ? a.q4_token_bytes : a.q2_token_bytes) + (4 * h + lg) * bs
-                               : (const uint8_t *)a.query;
-        const uint8_t *vp = ok ? kp + (a.component_values / 64) * bs : kp;
-        t.ks[i] = *(const uint16_t *)kp;
-        t.vs[i] = *(const uint16_t *)vp;
-        t.k[i][0] = *(const PtCodes *)(kp + 2);
-        t.v[i][0] = *(const PtCodes *)(vp + 2);
-        if (Q4) {
-            t.k[i][1] = *(const PtCodes *)(kp + (q4 ? 18 : 2));
-            t.v[i][1] = *(const PtCodes *)(vp + (q4 ? 18 : 2));
-        }
-        if (!ok) t.ks[i] = t.vs[i] = 0;
-    }
+// The pages of 64 tiles from `tile` on, one per lane (no tokens past T1 or the page table).
+__device__ __forceinline__ uint4 pt_descs(const GqaArgs &a, uint32_t tile, uint32_t T1, uint32_t lane) {
+    const uint32_t x = tile + lane, p = x < T1 ? x * 16 / a.page_tokens : a.page_count;
+    uint4 d = ((const uint4 *)a.desc)[p < a.page_count ? p : 0];
+    if (p >= a.page_count) d.x = d.z = 0;
+    return d;
 }
 
 // grid (splits, kv heads), 256 R threads, R = 1 or 2 tiles of 16 queries: waves 4 qt .. 4 qt + 3 serve
 // query tile qt (both quads read the keys, the first one's V codes are staged for both). A workgroup
 // takes tiles_per_wave tiles (a multiple of 16) from split * tiles_per_wave on.
-template <int R, int Q4>
-__device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T0, uint32_t T1, uint4 dnext, PtTiles &t) {
-    constexpr uint32_t RS = Q4 ? PT_RS4 : PT_RS2;
+// Q4: whether a tile of the workgroup lies in a Q4 page (tiles of Q2 pages are then widened).
+template <int R, bool Q4>
+__device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T0, uint32_t T1, uint4 desc) {
     const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t li = lane & 15, lg = lane >> 4, h = blockIdx.y, wave = wv & 3, qt = wv >> 2;
-    auto desc_of = [&](uint32_t tile) {  // lane i < 4: page of tile + i (no tokens past T1 or the page table)
-        const uint32_t x = tile + (lane & 3), p = x < T1 ? x * 16 / a.page_tokens : a.page_count;
-        const uint4 d = ((const uint4 *)a.desc)[p < a.page_count ? p : 0];
-        return p < a.page_count ? d : make_uint4(0, 0, 0, 0);
-    };
+    constexpr float inv_k = Q4 ? 1.0f / 15.0f : 1.0f / 3.0f;
+    constexpr int32_t neg_k = Q4 ? -15 : -3;
+    constexpr uint32_t blk = Q4 ? 32 : 16;  // bytes of a V block's codes
+    constexpr int N = Q4 ? 5 : 3;
     const uint32_t qi = 16 * qt + li;
     const int32_t lim = qi < a.queries ? (int32_t)(a.tokens - a.rows + qi / a.group) : -1;
-    const float qs = L.qs[qi];
     float m = -INFINITY, den = 0.0f;
-    int32_t xs[4];
     pa_v4f o[4];  // [dim tile]
 #pragma unroll
-    for (int b = 0; b < 4; b++) {
-        xs[b] = L.xs[qi][b];
-        o[b] = pa_v4f{0.0f, 0.0f, 0.0f, 0.0f};
-    }
+    for (int b = 0; b < 4; b++) o[b] = pa_v4f{0.0f, 0.0f, 0.0f, 0.0f};
+    uint8_t *kst = (uint8_t *)&L.p[qt][wave][0][0][0];
     for (uint32_t T = T0; T < T1; T += 16) {
-        const uint32_t tb = (T + 4 * wave) * 16;
+        const uint32_t tb = (T + 4 * wave) * 16, at = (T - T0) & 63;
+        if (T != T0 && at == 0) desc = pt_descs(a, T, T1, lane);
+        PtTiles t;
+        pt_tiles(a, desc, at + 4 * wave, t);
+        uint2 kr[4][N], vr[4][N];
+        auto load = [&](uint2 (&r)[4][N], uint32_t first) {  // first: of the token's blocks
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const bool q4 = Q4 && ((t.q4 >> i) & 1u);
+                pt_load<N, Q4 ? 17 : 9>(a, t.page[i], t.lo[i], t.hi[i], tb + 16 * i, first * (q4 ? 34 : 18),
+                                        q4 ? a.q4_token_bytes : a.q2_token_bytes, q4 ? 17 : 9, lane, r[i]);
+            }
+        };
+        load(kr, 4 * h);
+        if (qt == 0) load(vr, a.component_values / 64 + 4 * h);
         bool any = false;
         bool whole = tb + 63 + a.rows <= a.tokens;
 #pragma unroll
@@ -194,31 +233,36 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
             const uint32_t b = tb + 16 * i;
             any |= t.hi[i] > t.lo[i] && t.hi[i] > b && t.lo[i] < b + 16;
             whole = whole && t.lo[i] <= b && t.hi[i] >= b + 16;
-            if (Q4 && !((t.q4 >> i) & 1u)) {
-                pt_widen(t.k[i]);
-                pt_widen(t.v[i]);
-            }
         }
-        // ---- scales and V codes to LDS
-        uint32_t vmx = 0;
+        // ---- K and V by (token, block); scales and V codes to LDS
+        uint32_t kc[4][8];
+        auto stage = [&](uint8_t *rows, int i, const uint2 (&r)[N], uint32_t (&c)[8]) {
+            uint32_t sc;
+            const bool q4 = Q4 && ((t.q4 >> i) & 1u);
+            pt_stage<N, Q4 ? 17 : 9>(rows, q4 ? 34 : 18, lane, r, c, sc);
+            if (Q4 && !q4) pt_widen(c);
+            const uint32_t j = tb + 16 * i + li;
+            return pa_half(j >= t.lo[i] && j < t.hi[i] ? sc : 0u);  // absent tokens have a zero scale
+        };
 #pragma unroll
-        for (int i = 0; i < 4; i++) {
-            const float vs = pa_half(t.vs[i]);
-            vmx = max(vmx, __float_as_uint(vs) & 0x7fffffffu);  // (a NaN counts as the largest)
-            L.ksc[wv][i][lg][li] = pa_half(t.ks[i]) * (Q4 ? 1.0f / 15.0f : 1.0f / 3.0f);
-            if (qt) continue;
-            L.vsc[lg][64 * wave + 16 * i + li] = vs;
-            uint2 *d = (uint2 *)(L.v + (64 * wave + 16 * i + li) * RS + (Q4 ? 32 : 16) * lg);
+        for (int i = 0; i < 4; i++) L.ksc[wv][i][lg][li] = stage(kst, i, kr[i], kc[i]) * inv_k;
+        if (qt == 0) {
+            uint32_t vmx = 0;
 #pragma unroll
-            for (int x = 0; x < (Q4 ? 2 : 1); x++) {
-                d[2 * x] = make_uint2(t.v[i][x].x[0], t.v[i][x].x[1]);
-                d[2 * x + 1] = make_uint2(t.v[i][x].x[2], t.v[i][x].x[3]);
+            for (int i = 0; i < 4; i++) {
+                uint8_t *rows = L.v + (64 * wave + 16 * i) * PT_RS;
+                uint32_t c[8];
+                const float vs = stage(rows, i, vr[i], c);
+                vmx = max(vmx, __float_as_uint(vs) & 0x7fffffffu);  // (a NaN counts as the largest)
+                L.vsc[lg][64 * wave + 16 * i + li] = vs;
+                uint2 *d = (uint2 *)(rows + li * PT_RS + blk * lg);
+#pragma unroll
+                for (int x = 0; x < (Q4 ? 4 : 2); x++) d[x] = make_uint2(c[2 * x], c[2 * x + 1]);
             }
+            vmx = pt_row_umax(vmx);
+            if (li == 0) L.vmax[wave][lg] = vmx;
+            if (lane == 0) L.held[wave] = any;
         }
-#pragma unroll
-        for (int x = 1; x < 16; x <<= 1) vmx = max(vmx, (uint32_t)__shfl_xor((int)vmx, x));
-        if (qt == 0 && li == 0) L.vmax[wave][lg] = vmx;
-        if (qt == 0 && lane == 0) L.held[wave] = any;
         // ---- scores
         float s[4][4];
 #pragma unroll
@@ -232,43 +276,44 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
             asm volatile("" : "+v"(qoff));
 #pragma unroll
             for (int i = 0; i < 4; i++) {
-                uint32_t *k0 = t.k[i][0].x, *k1 = t.k[i][1].x;
                 if (Q4) {  // quarter q of a block is words 2 q, 2 q + 1
-                    uint32_t e0 = k0[0], e1 = k0[2], e2 = k1[0], e3 = k1[2], f0 = k0[1], f1 = k0[3], f2 = k1[1], f3 = k1[3];
-                    transpose4(e0, e1, e2, e3);
-                    transpose4(f0, f1, f2, f3);
-                    k0[0] = e0; k0[1] = e1; k0[2] = e2; k0[3] = e3;
-                    k1[0] = f0; k1[1] = f1; k1[2] = f2; k1[3] = f3;
+                    transpose4(kc[i][0], kc[i][2], kc[i][4], kc[i][6]);
+                    transpose4(kc[i][1], kc[i][3], kc[i][5], kc[i][7]);
                 } else {
-                    transpose4(k0[0], k0[1], k0[2], k0[3]);
+                    transpose4(kc[i][0], kc[i][1], kc[i][2], kc[i][3]);
                 }
             }
 #pragma unroll
             for (int b = 0; b < 4; b++) {
                 __builtin_amdgcn_sched_barrier(0);  // (a block's results at a time in registers)
-                pa_i4 qv[3];
+                pa_i4 qv[3], ak[4];
+                if (Q4) {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t x = kc[i][2 * b], y = kc[i][2 * b + 1];
+                        const uint32_t xl = (x << 1) & 0x1E1E1E1Eu, xh = (x >> 3) & 0x1E1E1E1Eu;
+                        const uint32_t yl = (y << 1) & 0x1E1E1E1Eu, yh = (y >> 3) & 0x1E1E1E1Eu;
+                        ak[i] = pa_i4{(int)__builtin_amdgcn_perm(yl, xl, 0x06040200u), (int)__builtin_amdgcn_perm(yh, xh, 0x06040200u),
+                                      (int)__builtin_amdgcn_perm(yl, xl, 0x07050301u), (int)__builtin_amdgcn_perm(yh, xh, 0x07050301u)};
+                    }
+                } else {
+#pragma unroll
+                    for (int i = 0; i < 4; i++) {
+                        const uint32_t x = kc[i][b];
+                        ak[i] = pa_i4{(int)((x << 1) & 0x06060606u), (int)((x >> 1) & 0x06060606u), (int)((x >> 3) & 0x06060606u),
+                                      (int)((x >> 5) & 0x06060606u)};
+                    }
+                }
+                const int32_t c0 = neg_k * L.xs[qi][b];
 #pragma unroll
                 for (int k = 0; k < 3; k++) qv[k] = *(const pa_i4 *)(&L.limbs[k][0][64 * b] + qoff);
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    pa_i4 ak;
-                    if (Q4) {
-                        const uint32_t x = t.k[i][0].x[b], y = t.k[i][1].x[b];
-                        const uint32_t xl = (x << 1) & 0x1E1E1E1Eu, xh = (x >> 3) & 0x1E1E1E1Eu;
-                        const uint32_t yl = (y << 1) & 0x1E1E1E1Eu, yh = (y >> 3) & 0x1E1E1E1Eu;
-                        ak = pa_i4{(int)__builtin_amdgcn_perm(yl, xl, 0x06040200u), (int)__builtin_amdgcn_perm(yh, xh, 0x06040200u),
-                                   (int)__builtin_amdgcn_perm(yl, xl, 0x07050301u), (int)__builtin_amdgcn_perm(yh, xh, 0x07050301u)};
-                    } else {
-                        const uint32_t x = t.k[i][0].x[b];
-                        ak = pa_i4{(int)((x << 1) & 0x06060606u), (int)((x >> 1) & 0x06060606u), (int)((x >> 3) & 0x06060606u),
-                                   (int)((x >> 5) & 0x06060606u)};
-                    }
                     const float4 f = *(const float4 *)&L.ksc[wv][i][b][4 * lg];
                     const float fb[4] = {f.x, f.y, f.z, f.w};
-                    const int32_t c0 = (Q4 ? -15 : -3) * xs[b];
-                    const pa_i4 a0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak, qv[0], pa_i4{c0, c0, c0, c0}, 0, 0, 0);
-                    const pa_i4 a1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak, qv[1], pa_i4{0, 0, 0, 0}, 0, 0, 0);
-                    const pa_i4 a2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak, qv[2], pa_i4{0, 0, 0, 0}, 0, 0, 0);
+                    const pa_i4 a0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak[i], qv[0], pa_i4{c0, c0, c0, c0}, 0, 0, 0);
+                    const pa_i4 a1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak[i], qv[1], pa_i4{0, 0, 0, 0}, 0, 0, 0);
+                    const pa_i4 a2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak[i], qv[2], pa_i4{0, 0, 0, 0}, 0, 0, 0);
 #pragma unroll
                     for (int c = 0; c < 4; c++) {
                         const uint32_t u = (uint32_t)a0[c] + ((uint32_t)a1[c] << 8) + ((uint32_t)a2[c] << 16);
@@ -279,6 +324,7 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
         }
         float mt = -INFINITY;
         if (any) {
+            const float qs = L.qs[qi];
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
@@ -301,14 +347,6 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
         }
         mt = pa_max_x32(pa_max_x16(mt));
         if (lg == 0) L.smax[wave][qt][li] = mt;
-        // The next step's loads go out while this one's probabilities are
-        // exchanged (Q4's, twice the registers, after the value product).
-        const bool more = T + 16 < T1;
-        auto next = [&] {
-            pt_load<Q4>(a, dnext, (T + 16 + 4 * wave) * 16, h, li, lg, t);
-            dnext = desc_of(T + 32 + 4 * wave);
-        };
-        if (!Q4 && more) next();
         lds_barrier();
         float mn = m;
 #pragma unroll
@@ -334,7 +372,7 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
         const int ex = min(max((int)(vb >> 23) - 126, -24), 17);  // fp16 scales below 2^ex
         const float sc = ldexpf(1.0f, 22 - ex);
         const float back = vb < 0x7f800000u ? ldexpf(1.0f, ex - 22) : __builtin_nanf("");
-        const uint32_t vrow = (16 * (li >> 2) + 4 * lg + (li & 3)) * RS;
+        const uint32_t vrow = (16 * (li >> 2) + 4 * lg + (li & 3)) * PT_RS + blk * wave;
         pa_i4 acc[4][3], ones[3];
 #pragma unroll
         for (int k = 0; k < 3; k++) {
@@ -367,29 +405,39 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
                 ones[k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(pa_i4{0x01010101, 0x01010101, 0x01010101, 0x01010101}, bl[k],
                                                                 ones[k], 0, 0, 0);
             }
-            const uint8_t *vbase = L.v + 64 * w * RS + vrow + (Q4 ? 32 : 16) * wave;
+            const uint8_t *vbase = L.v + 64 * w * PT_RS + vrow;
+            auto read = [&](int j) {
+                return __builtin_amdgcn_ds_read_tr4_b64_v2i32((__attribute__((address_space(3))) pt_v2i *)(vbase + 8 * j));
+            };
+            pa_i4 av[4];
+            if (Q4) {
 #pragma unroll
-            for (int j = 0; j < (Q4 ? 4 : 2); j++) {
-                const pt_v2i x = __builtin_amdgcn_ds_read_tr4_b64_v2i32(
-                    (__attribute__((address_space(3))) pt_v2i *)(vbase + 8 * j));
-                const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1];
+                for (int d = 0; d < 4; d++) {
+                    const pt_v2i x = read(d);
+                    av[d] = pa_i4{x[0] & 0x0F0F0F0F, (int)((uint32_t)x[0] >> 4) & 0x0F0F0F0F, x[1] & 0x0F0F0F0F,
+                                  (int)((uint32_t)x[1] >> 4) & 0x0F0F0F0F};
+                }
+            } else {
 #pragma unroll
-                for (int par = 0; par < (Q4 ? 1 : 2); par++) {
-                    const uint32_t mask = Q4 ? 0x0F0F0F0Fu : 0x03030303u;
-                    const pa_i4 av = {(int)((x0 >> (2 * par)) & mask), (int)((x0 >> (4 + 2 * par)) & mask),
-                                      (int)((x1 >> (2 * par)) & mask), (int)((x1 >> (4 + 2 * par)) & mask)};
-                    const int d = Q4 ? j : 2 * j + par;
-#pragma unroll
-                    for (int k = 0; k < 3; k++)
-                        acc[d][k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av, bl[k], acc[d][k], 0, 0, 0);
+                for (int j = 0; j < 2; j++) {
+                    const pt_v2i x = read(j);
+                    const uint32_t x0 = (uint32_t)x[0], x1 = (uint32_t)x[1];
+                    av[2 * j] = pa_i4{(int)(x0 & 0x03030303u), (int)((x0 >> 4) & 0x03030303u), (int)(x1 & 0x03030303u),
+                                      (int)((x1 >> 4) & 0x03030303u)};
+                    av[2 * j + 1] = pa_i4{(int)((x0 >> 2) & 0x03030303u), (int)((x0 >> 6) & 0x03030303u),
+                                          (int)((x1 >> 2) & 0x03030303u), (int)((x1 >> 6) & 0x03030303u)};
                 }
             }
+#pragma unroll
+            for (int d = 0; d < 4; d++)
+#pragma unroll
+                for (int k = 0; k < 3; k++)
+                    acc[d][k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[d], bl[k], acc[d][k], 0, 0, 0);
         }
-        if (Q4 && more) next();
-        const float f = back * (Q4 ? 1.0f / 15.0f : 1.0f / 3.0f);
+        const float f = back * inv_k;
         int32_t n[3];
 #pragma unroll
-        for (int k = 0; k < 3; k++) n[k] = (Q4 ? -15 : -3) * ones[k][0];
+        for (int k = 0; k < 3; k++) n[k] = neg_k * ones[k][0];
 #pragma unroll
         for (int d = 0; d < 4; d++)
 #pragma unroll
@@ -429,36 +477,17 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
 template <int R>
 __device__ __forceinline__ void paged_gqa_tiles(const GqaArgs &a) {
     __shared__ __align__(16) PtLds<R> L;
-    const uint32_t lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3;
-    const uint32_t li = lane & 15, lg = lane >> 4, h = blockIdx.y;
+    const uint32_t lane = threadIdx.x & 63;
     const uint32_t T0 = blockIdx.x * a.tiles_per_wave, T1 = min(T0 + a.tiles_per_wave, a.tiles);
-    // Any Q4 page in the workgroup's range? (lanes stride over its tiles)
-    bool q4 = false;
-    for (uint32_t x = T0 + lane; x < T1; x += 64) {
-        const uint32_t p = x * 16 / a.page_tokens;
-        q4 = q4 || (p < a.page_count && a.desc[p].precision != 0);
-    }
-    auto desc_of = [&](uint32_t tile) {
-        const uint32_t x = tile + (lane & 3), p = x < T1 ? x * 16 / a.page_tokens : a.page_count;
-        const uint4 d = ((const uint4 *)a.desc)[p < a.page_count ? p : 0];
-        return p < a.page_count ? d : make_uint4(0, 0, 0, 0);
-    };
-    const uint4 d0 = desc_of(T0 + 4 * wave), d1 = desc_of(T0 + 16 + 4 * wave);
+    const uint4 desc = pt_descs(a, T0, T1, lane);
     float qv[1][16];
-    pa_prep_load<1>(a, h, qv);
-    PtTiles t;
-    // The first step's loads are in flight while the queries are split.
-    if (__builtin_amdgcn_ballot_w64(q4) == 0) {
-        pt_load<0>(a, d0, (T0 + 4 * wave) * 16, h, li, lg, t);
-        pt_prep<R>(a, qv[0], L);
-        lds_barrier();
-        pt_run<R, 0>(a, L, T0, T1, d1, t);
-    } else {
-        pt_load<1>(a, d0, (T0 + 4 * wave) * 16, h, li, lg, t);
-        pt_prep<R>(a, qv[0], L);
-        lds_barrier();
-        pt_run<R, 1>(a, L, T0, T1, d1, t);
-    }
+    pa_prep_load<1>(a, blockIdx.y, qv);
+    bool q4 = desc.x != 0;
+    for (uint32_t T = T0 + 64; T < T1; T += 64) q4 = q4 || pt_descs(a, T, T1, lane).x != 0;
+    pt_prep<R>(a, qv[0], L);
+    lds_barrier();
+    if (__builtin_amdgcn_ballot_w64(q4) == 0) pt_run<R, false>(a, L, T0, T1, desc);
+    else pt_run<R, true>(a, L, T0, T1, desc);
 }
 
 extern "C" __global__ __launch_bounds__(256, 2) void ctox_paged_gqa_tiles_r1_gfx950(GqaArgs a) { paged_gqa_tiles<1>(a); }
