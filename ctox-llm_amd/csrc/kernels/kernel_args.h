@@ -527,7 +527,7 @@ struct GqaArgs {
     uint32_t q2_token_bytes;
     uint32_t q4_token_bytes;
     uint32_t tiles;          // ceil(tokens / 16)
-    uint32_t tiles_per_wave; // page-aligned tiles: per workgroup, a multiple of 16
+    uint32_t tiles_per_wave; // (ctox_paged_gqa_tiles: per workgroup, a multiple of 16)
     uint32_t splits;
     float scale;
     uint32_t tile_pages;     // 1 when page_tokens % 16 == 0: a 16-token tile lies in one page

@@ -1,7 +1,7 @@
-// Split-KV attention over page-aligned tiles (page_tokens a multiple of 16):
-// both products on int8 MFMA 16x16x64 with exact integer sums. Included after
-// paged_attention.hip (page format and the other page sizes' kernel) and
-// qmatvec_tiled.hip (transpose4).
+// Split-KV attention over page-aligned tiles (page_tokens a multiple of 16) for
+// contexts that fill the CUs: both products on int8 MFMA 16x16x64 with exact
+// integer sums. Included after paged_attention.hip (page format, the kernels of
+// smaller contexts and other page sizes) and qmatvec_tiled.hip (transpose4).
 //
 // A workgroup takes one KV head and a run of 256-token steps; wave w loads and
 // scores tokens 64 w .. 64 w + 63 of a step (four 16-token tiles), and then
@@ -30,12 +30,16 @@
 //  sum X code and sum X (a row of ones) give sum X (2 code - K), one conversion
 //  per limb and one fma per step.
 //
-// The other split, a wave keeping its tokens for both products (as the fp32
-// kernel does), pays the O conversion per wave and merges four O's in LDS; here
+// The other split, a wave keeping its tokens for both products (as the other
+// kernels do), pays the O conversion per wave and merges four O's in LDS; here
 // one step's 256 tokens are converted once.
 //
-// Bound by VALU issue: about 1200 instructions per wave and 256-token step (the
-// f16-MFMA kernel before took 750 per 16-token tile, 3000 for the same tokens).
+// Bound by VALU issue and a long start: 1900 VALU instructions per wave and step
+// (the f16 kernel takes 750 per 16-token tile, 3000 for the same tokens), but
+// every wave scores four tiles before the first result. 32768 tokens of 24 / 4
+// heads: 5 rows 30.1 us against 39.5, 1 row 19.8 against 21.3 (the combine's 3 us
+// included). Against float64 the output is off by 1.8e-6 of its norm, 2.4e-5
+// with f16 codes and a separate sum of P x scale.
 
 typedef int pt_v2i __attribute__((ext_vector_type(2)));
 #define PT_STEP 256   // tokens per step
@@ -365,13 +369,18 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
             *(float4 *)&L.p[qt][wave][i][lane][0] = p;
         }
         den = den * alpha + sum;
-        lds_barrier();
-        // ---- O^T of value block `wave` over the step's tokens
+        // Value block `wave`: its scales times 2^(22 - e), 2^e above the largest (fp16 scales).
         uint32_t vb = max(max(L.vmax[0][wave], L.vmax[1][wave]), max(L.vmax[2][wave], L.vmax[3][wave]));
         vb = __builtin_amdgcn_readfirstlane(vb);
-        const int ex = min(max((int)(vb >> 23) - 126, -24), 17);  // fp16 scales below 2^ex
-        const float sc = ldexpf(1.0f, 22 - ex);
+        const int ex = min(max((int)(vb >> 23) - 126, -24), 17);
         const float back = vb < 0x7f800000u ? ldexpf(1.0f, ex - 22) : __builtin_nanf("");
+        if (qt == 0) {
+            float4 *v = (float4 *)&L.vsc[wave][4 * lane];
+            const float sc = ldexpf(1.0f, 22 - ex);
+            *v = make_float4(v->x * sc, v->y * sc, v->z * sc, v->w * sc);
+        }
+        lds_barrier();
+        // ---- O^T of the block over the step's tokens
         const uint32_t vrow = (16 * (li >> 2) + 4 * lg + (li & 3)) * PT_RS + blk * wave;
         pa_i4 acc[4][3], ones[3];
 #pragma unroll
@@ -390,7 +399,7 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
                 const float pp[4] = {p.x, p.y, p.z, p.w}, vv[4] = {v.x, v.y, v.z, v.w};
                 // The sum's low mantissa bits are X + 2^22; + 0x408080 makes it X + 0x808080 (low 24 bits).
 #pragma unroll
-                for (int c = 0; c < 4; c++) z[4 * i + c] = __float_as_uint(fmaf(pp[c], vv[c] * sc, 12582912.0f)) + 0x408080u;
+                for (int c = 0; c < 4; c++) z[4 * i + c] = __float_as_uint(fmaf(pp[c], vv[c], 12582912.0f)) + 0x408080u;
             }
             uint32_t l[3][4];
 #pragma unroll
@@ -435,16 +444,15 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
                     acc[d][k] = __builtin_amdgcn_mfma_i32_16x16x64_i8(av[d], bl[k], acc[d][k], 0, 0, 0);
         }
         const float f = back * inv_k;
-        int32_t n[3];
-#pragma unroll
-        for (int k = 0; k < 3; k++) n[k] = neg_k * ones[k][0];
+        const int32_t n01 = neg_k * (ones[0][0] + (ones[1][0] << 8)), n2 = neg_k * ones[2][0];
 #pragma unroll
         for (int d = 0; d < 4; d++)
 #pragma unroll
             for (int c = 0; c < 4; c++) {
-                const float t0 = (float)(2 * acc[d][0][c] + n[0]), t1 = (float)(2 * acc[d][1][c] + n[1]);
-                const float t2 = (float)(2 * acc[d][2][c] + n[2]);
-                o[d][c] = fmaf(fmaf(t2, 65536.0f, fmaf(t1, 256.0f, t0)), f, o[d][c] * alpha);
+                // The low two limbs' sums are below 2^20: joined in int32.
+                const float t01 = (float)(2 * (acc[d][0][c] + (acc[d][1][c] << 8)) + n01);
+                const float t2 = (float)(2 * acc[d][2][c] + n2);
+                o[d][c] = fmaf(fmaf(t2, 65536.0f, t01), f, o[d][c] * alpha);
             }
         lds_barrier();  // the step's LDS is free
     }

@@ -148,6 +148,42 @@ def test_paged_attention_peaked_scores(hip):
     np.testing.assert_allclose(out.cpu().numpy(), want, rtol=1e-3, atol=1e-4 * float(np.abs(want).max()))
 
 
+# Contexts whose 256-token steps fill the CUs (int8 MFMA for both products). 4 KV heads on 256 CUs: from 17
+# steps with more than 16 queries, 57 .. 64 and 121 .. 128 with fewer; 16500 tokens of 5 rows: two steps per
+# workgroup.
+@pytest.mark.parametrize("tokens,rows,page,sink,recent,special", [
+    (4353, 5, 16, 16, 16, False),      # the last step holds one token; the first mixes Q4 and Q2 pages
+    (4600, 3, 32, 288, 64, True),      # 18 queries; an infinite value scale
+    (16500, 5, 128, 128, 256, False),
+    (14337, 1, 16, 0, 16, False), (16384, 2, 16, 48, 512, True),
+])
+def test_paged_attention_long(hip, tokens, rows, page, sink, recent, special):
+    say(f"case paged attention long tokens={tokens} rows={rows} page={page}")
+    rng = np.random.default_rng(tokens + rows)
+    dev, ref = make_caches(hip, tokens + 8, page, sink, recent)
+    cv = KVH * HD
+    k = (rng.standard_normal((tokens, cv)) * 1.5).astype(np.float32)
+    v = rng.standard_normal((tokens, cv)).astype(np.float32)
+    push_both(dev, ref, k, v)
+    if special:  # an infinite value scale in a page that stays Q4 (the oracle takes finite values only)
+        at = dev.q4_pool.view(-1)[2 * dev.params(QH).q4_token_bytes + (cv + HD + 128) // 64 * 34:]
+        at[:2] = torch.tensor([0x00, 0x7C], dtype=torch.uint8, device="cuda")
+    q = (rng.standard_normal((rows, QH, HD)) * 1.5).astype(np.float32)
+    out = dev.attention(torch.from_numpy(q).cuda(), rows, QH)
+    torch.cuda.synchronize()
+    got = out.cpu().numpy()
+    want = pk.paged_attention(ref, q, rows, QH, KVH, HD).reshape(rows, QH, HD)
+    finite = np.ones(want.shape, bool)
+    if special:  # that block of the queries of KV head 1
+        finite[:, QH // KVH:2 * QH // KVH, 128:192] = False
+    assert np.array_equal(np.isfinite(got), finite)
+    # A query rounded at 2^-22 of its row's largest (6 of 1.5 sigma 1.5) moves a score by at most
+    # scale * sum |k| * 6 * 1.5 * 2^-22 = 1/16 * 256 * 1.2 * 9 * 2^-22 = 4e-5, a probability by that part of
+    # itself and the output by twice that of sum p |v|, about 1: 8e-5 (the values' 2^-23 and the sums' int32
+    # are far below).
+    np.testing.assert_allclose(got[finite], want[finite], rtol=0, atol=8e-5)
+
+
 def test_paged_attention_errors(hip):
     import ctox_hip
     from ctox_hip.paged_kv import DevicePagedKvCache
