@@ -7,20 +7,20 @@
 // G_t = sum_{s<=t} log_decay_s (relative to the chunk start) and g_t = exp(G_t):
 //   S_t = g_t S_0 + sum_{r<=t} exp(G_t - G_r) k_r d_r^T
 //   d_s = b_s (v_s - g_s S_0^T k_s - sum_{r<s} exp(G_s - G_r) (k_s.k_r) d_r).
-// With L the strictly lower b_s (k_s.k_r) and T0 = (I + L)^{-1} (no decay: the
-// decayed inverse is diag(g) T0 diag(1/g)), this is
-//   D   = U - diag(g) W S_0,   W = T0 diag(b) K,
-//                              U[s] = sum_{r<=s} exp(G_s - G_r) T0[s][r] b_r v_r
+// With L the strictly lower b_s exp(G_s - G_r) (k_s.k_r) and T = (I + L)^{-1},
+// this is
+//   D   = U - W S_0,   U = T diag(b) V,   W = T diag(b g) K
 //   O   = diag(g) Q S_0 + A D,       A[t][r] = exp(G_t - G_r) (q_t.k_r), r <= t
 //   S_C = g_C S_0 + sum_r exp(G_C - G_r) k_r d_r^T.
 // Every decay factor is exp of a non-positive difference for decays <= 1, so
-// nothing overflows however strong the decay. Only D and S_C depend on the
+// nothing overflows however strong the decay. (The decay belongs in the
+// inverse: that of the undecayed I + L grows as (beta - 1)^n for beta > 2.) Only D and S_C depend on the
 // chunks before, so all of W, U, A and the scaled rows of Q and K are made for
 // every chunk in parallel (pass 1) and the sequential pass 2 is two small
 // products deep per chunk.
 //
 // Pass 1 (ctox_gdn_chunk_prep_gfx950, one workgroup per (head, chunk)): fp32
-// MFMA throughout; T0 by blocks: the four 16 x 16 diagonal blocks by forward
+// MFMA throughout; T by blocks: the four 16 x 16 diagonal blocks by forward
 // substitution (a wave each), the blocks below them on MFMA one block row at a
 // time. Its matrices leave as MFMA operands, see below.
 // Pass 2 (ctox_gdn_chunk_scan{1,2}_gfx950, one workgroup per (head, 16 or 32
@@ -33,7 +33,7 @@
 // lo hi, fp32 accumulation): 16 times the fp32 MFMA rate for 22 significant
 // bits, at or under the fp32 products' own rounding (measured below). The
 // split is kept inside f16's range by powers of two that cost nothing: the
-// operands of pass 1 are scaled by 2^14 over their row's norm (which a factor
+// operands of pass 1 are scaled by 2^14 over their row's largest magnitude (which a factor
 // on the product's rows undoes), the state by 2^15 over each column's largest
 // magnitude per 32 keys, D by 2^15 over a bound of its column's (its operand
 // may be up to 2^10 below the bound before a bit is lost). fp32 inputs of any
@@ -183,15 +183,15 @@ __device__ __forceinline__ gv4f load4(const float *row, uint32_t col, uint32_t w
 // exchanges around 320 fp32 MFMAs per wave (18 us alone on a CU, 13 us of the
 // CU's time each when three share it; without its stores 10% less, without W's
 // and U's products no less). K, Q and V are requested up front, Q stays in
-// registers and V waits in them for K's LDS rows, T0 replaces L in place, so
-// 52 KB of LDS let three workgroups share a CU (two with Q and T0 in LDS: 63
+// registers and V waits in them for K's LDS rows, T replaces L in place, so
+// 52 KB of LDS let three workgroups share a CU (two with Q and T in LDS: 63
 // against 43 us for the 640 workgroups of 20 chunks of 32 heads).
 template <bool VEC>
 __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     __shared__ __align__(16) float kh[GC * SPAD];  // raw K rows, then V rows
-    __shared__ float tt[GC * TPAD];                // L, T0, W's and then U's left operand
+    __shared__ float tt[GC * TPAD];                // L, T, W's and then U's left operand
     __shared__ __align__(16) float G[GC], bt[GC], kinv_s[GC], ekf[GC];
-    __shared__ float wsq[4][GC];
+    __shared__ float wmax[4][GC];
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t m16 = lane & 15, g = lane >> 4;
     // A token's heads lie side by side, so the workgroups of one XCD (block % 8)
@@ -284,7 +284,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
             if (u > w) acc[u] = tile_rows(krow + 16 * (u - w - 1) * SPAD, ks);
     }
     {   // A: row t = own, this lane's r = 16 u + 4 g + x
-        float sq = 0.0f;
+        float mx = 0.0f;
         const float Gown = G[own];
 #pragma unroll
         for (uint32_t u = 0; u < 4; u++) {
@@ -295,10 +295,10 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
                 const uint32_t r = 16 * u + 4 * g + x;
                 const float val = r <= own ? exp_decay(Gown - Gr[x]) * (kr4[x] * qinv) * acc[u][x] : 0.0f;
                 acc[u][x] = val;
-                sq += val * val;
+                mx = fmaxf(mx, fabsf(val));
             }
         }
-        const int e = exponent_of(sqrtf(groups_sum(sq)));
+        const int e = exponent_of(groups_max(mx));  // (squares of large entries would overflow)
         const float sc = pow2(14 - e);
         if (g == 0) aux[128 + own] = qscale * pow2(e - 14);
         uint4 *dst = (uint4 *)(base + GF_A) + w * 256 + lane;
@@ -313,20 +313,20 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     }
     {   // L of strip 3 - w, strictly lower: the tile's rows are r, its columns s
         const uint32_t s = 16 * (3 - w) + m16;
-        const float f = bt[s] * kinv_s[s];
+        const float f = bt[s] * kinv_s[s], Gs = G[s];
 #pragma unroll
         for (uint32_t u = 1; u < 5; u++) {
             if (u <= w) continue;
-            const gv4f kr4 = *(const gv4f *)&kinv_s[16 * (u - w - 1) + 4 * g];
+            const gv4f kr4 = *(const gv4f *)&kinv_s[16 * (u - w - 1) + 4 * g], Gr = *(const gv4f *)&G[16 * (u - w - 1) + 4 * g];
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 const uint32_t r = 16 * (u - w - 1) + 4 * g + x;
-                tt[s * TPAD + r] = r < s ? f * kr4[x] * acc[u][x] : 0.0f;
+                tt[s * TPAD + r] = r < s ? exp_decay(Gs - Gr[x]) * (f * kr4[x]) * acc[u][x] : 0.0f;
             }
         }
     }
     lds_barrier();
-    // T0 = (I + L)^{-1} over L, blockwise over 16 x 16 blocks:
+    // T = (I + L)^{-1} over L, blockwise over 16 x 16 blocks:
     //   T_ii = (I + L_ii)^{-1}                   forward substitution, wave i
     //                                            (row s of L is last read for row s of T);
     //   T_ij = -T_ii sum_{k=j}^{i-1} L_ik T_kj   block row i after row i - 1,
@@ -391,17 +391,17 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         }
     }
     lds_barrier();
-    // tt: T0 diag(b kinv) (W's left operand, on the raw K rows); in registers,
-    // for tt later: the decayed T0 diag(b) (U's). Lane: column r, rows 16 w + i.
+    // tt: T diag(b g kinv) (W's left operand, on the raw K rows); in registers,
+    // for tt later: T diag(b) (U's). Lane: column r, rows 16 w + i.
     // Blocks above the diagonal are read by no product.
     float tu[16];
     {
-        const float b = bt[lane], ki = kinv_s[lane];
+        const float b = bt[lane], ki = kinv_s[lane] * expf(gl);
 #pragma unroll
         for (int i = 0; i < 16; i++) {
             const uint32_t s = 16 * w + i;
             const float t = tt[s * TPAD + lane] * b;
-            tu[i] = lane <= s ? t * exp_decay(G[s] - gl) : 0.0f;
+            tu[i] = t;
             tt[s * TPAD + lane] = t * ki;
         }
     }
@@ -425,11 +425,11 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         }
 #pragma unroll
     for (int st = 0; st < 4; st++) {
-        float sq = 0.0f;
+        float mx = 0.0f;
 #pragma unroll
-        for (int x = 0; x < 4; x++) sq += wt[st][0][x] * wt[st][0][x] + wt[st][1][x] * wt[st][1][x];
-        sq = groups_sum(sq);
-        if (g == 0) wsq[w][16 * st + m16] = sq;
+        for (int x = 0; x < 4; x++) mx = fmaxf(mx, fmaxf(fabsf(wt[st][0][x]), fabsf(wt[st][1][x])));
+        mx = groups_max(mx);
+        if (g == 0) wmax[w][16 * st + m16] = mx;
     }
     lds_barrier();  // K rows and W's left operand are dead
 #pragma unroll
@@ -441,7 +441,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
 #pragma unroll
         for (int st = 0; st < 4; st++) {
             const uint32_t s = 16 * st + m16;
-            const int e = exponent_of(sqrtf((wsq[0][s] + wsq[1][s]) + (wsq[2][s] + wsq[3][s])));
+            const int e = exponent_of(fmaxf(fmaxf(wmax[0][s], wmax[1][s]), fmaxf(wmax[2][s], wmax[3][s])));
             const float sc = pow2(14 - e);
             uint4 f[2];
             split8(wt[st][0] * sc, wt[st][1] * sc, f);
@@ -451,10 +451,10 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     }
     if (w == 0) {
         const float ge = expf(gl);
-        const float nw = sqrtf((wsq[0][lane] + wsq[1][lane]) + (wsq[2][lane] + wsq[3][lane]));
-        aux[lane] = ge * pow2(exponent_of(nw) - 14);
+        const float nw = fmaxf(fmaxf(wmax[0][lane], wmax[1][lane]), fmaxf(wmax[2][lane], wmax[3][lane]));
+        aux[lane] = pow2(exponent_of(nw) - 14);
         aux[64 + lane] = qscale * ge * pow2(-14);
-        float wn = ge * nw;
+        float wn = nw;
 #pragma unroll
         for (int o = 32; o > 0; o >>= 1) wn = fmaxf(wn, __shfl_xor(wn, o));
         if (lane == GC - 1) {
@@ -538,10 +538,10 @@ __device__ __forceinline__ gv4f times_state(const uint4 (&x)[4][2], const GdnSca
     return (acc[0] * sf[0] + acc[1] * sf[1]) + (acc[2] * sf[2] + acc[3] * sf[3]);
 }
 
-// Exponent of D's scale: |D| <= max|U| + max_s |g_s W_s| |S column|, and a
-// key step's 32 values are below sf 2^15 each.
+// Exponent of D's scale: |D| <= max|U| + max|W| sum|S column|, and a key
+// step's 32 values are below sf 2^15 each.
 __device__ __forceinline__ int d_exponent(float mu, float wn, const float (&sf)[4]) {
-    return exponent_of(mu + wn * (32768.0f * 5.66f) * ((sf[0] + sf[1]) + (sf[2] + sf[3])));
+    return exponent_of(mu + wn * (32768.0f * 32.0f) * ((sf[0] + sf[1]) + (sf[2] + sf[3])));
 }
 
 // NT: value tiles (of 16 columns) per workgroup.

@@ -125,6 +125,25 @@ def test_chunked_prefill_magnitudes(hip, orc, heads, dv, vs, ss, bmax, ldmax):
     close(st_gpu, st_ref, 1e-4, "state")
 
 
+@pytest.mark.parametrize("beta,ld", [(6.0, -3.0), (3.2, -0.01)])
+def test_chunked_prefill_repeated_key(hip, orc, beta, ld):
+    """A repeated key with beta above 2: the undecayed I + L has an inverse of
+    (beta - 1)^n, past fp32 at 6 although the decayed one and the outputs stay
+    small; at 3.2 with little decay the state itself grows to 1e20."""
+    T, heads, dk, dv = 64, 2, 128, 64
+    say(f"case gdn repeated key beta={beta} ld={ld}")
+    q, k, v, lds, be = gdn_inputs(T, heads, heads, dk, dv, 21)
+    k = np.repeat(k[:1], T, axis=0)
+    lds, be = np.full_like(lds, ld), np.full_like(be, beta)
+    st_ref = (np.random.default_rng(T).standard_normal(heads * dk * dv) * 0.1).astype(np.float32)
+    st_gpu = st_ref.copy()
+    ref = orc.gated_delta_sequence(q, k, v, lds, be, st_ref, T, heads, dk, dv)
+    got = hip.gated_delta_sequence(q, k, v, lds, be, st_gpu, T, heads, dk, dv, 64)
+    assert np.all(np.isfinite(ref))
+    close(got, ref, 1e-3, "output")
+    close(st_gpu, st_ref, 1e-4, "state")
+
+
 @pytest.mark.parametrize("T", [1024, 4096])
 def test_chunked_prefill_long(hip, orc, T):
     """BASELINE config 4 shapes through the chunk-64 path, up to the config's
