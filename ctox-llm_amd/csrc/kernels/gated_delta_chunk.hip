@@ -14,9 +14,9 @@
 //   S_C = g_C S_0 + sum_r exp(G_C - G_r) k_r d_r^T.
 // Every decay factor is exp of a non-positive difference for decays <= 1, so
 // nothing overflows however strong the decay. (The decay belongs in the
-// inverse: that of the undecayed I + L grows as (beta - 1)^n for beta > 2.) Only D and S_C depend on the
-// chunks before, so all of W, U, A and the scaled rows of Q and K are made for
-// every chunk in parallel (pass 1) and the sequential pass 2 is two small
+// inverse: that of the undecayed I + L grows as (beta - 1)^n for beta > 2.)
+// Only D and S_C depend on the chunks before, so all of W, U, A and the scaled
+// rows of Q and K are made for every chunk in parallel (pass 1) and the sequential pass 2 is two small
 // products deep per chunk.
 //
 // Pass 1 (ctox_gdn_chunk_prep_gfx950, one workgroup per (head, chunk)): fp32
@@ -28,16 +28,13 @@
 // need no exchange. Padded tokens of a partial chunk have k = q = v = 0,
 // beta = 0 and log_decay = 0: identity steps.
 //
-// Pass 2's products run on v_mfma_f32_16x16x32_f16 with every operand split
-// into an f16 high and low part (three MFMAs per product: hi hi + hi lo +
-// lo hi, fp32 accumulation): 16 times the fp32 MFMA rate for 22 significant
-// bits, at or under the fp32 products' own rounding (measured below). The
-// split is kept inside f16's range by powers of two that cost nothing: the
-// operands of pass 1 are scaled by 2^14 over their row's largest magnitude (which a factor
-// on the product's rows undoes), the state by 2^15 over each column's largest
-// magnitude per 32 keys, D by 2^15 over a bound of its column's (its operand
-// may be up to 2^10 below the bound before a bit is lost). fp32 inputs of any
-// magnitude therefore keep their precision.
+// Pass 2's products run on v_mfma_f32_16x16x32_bf16 with every operand as the
+// exact sum of three bf16 parts (24 significant bits, fp32's exponents: no
+// scales, whatever the magnitudes of neighbouring tokens, keys or columns are)
+// and the six products of parts above 2^-24, accumulated in fp32: 2.7 times the
+// fp32 MFMA rate. (Two f16 parts under powers of two per row and column take
+// half the MFMAs, but elements 2^17 below their row's or column's largest lose
+// bits that fp32 keeps.)
 //
 // Pass 2 is a latency chain: per chunk the state operand, W S_0, D, its
 // exchange, K^T D. Four waves hold the state (fp32, in registers: wave w rows
@@ -45,15 +42,18 @@
 // them from the same two exchanges. The contraction index order of an operand
 // is free as long as both sides agree, and it is chosen so that a lane's MFMA
 // results are the very elements of its next operand: no transposes. Nothing
-// but the 8 KB state and 4 KB D operands passes through LDS; pass 1's operands
+// but the 12 KB state and 6 KB D operands passes through LDS; pass 1's operands
 // are read from memory in fragment order, one chunk ahead, straight to
-// registers, a few at a time between the chunk's products: 120 KB per chunk and
-// CU take 0.8 us of the CU's load path, which issued in one go came on top of
-// the products' 1.2 us (20 chunks of 32 heads 40.9, interleaved 35.3 us).
-// 4096 tokens of 32 heads: 227 us, against 372 for the same chunk algorithm with
-// all of T (b V - b g K S_0), Q S_0 + A D and the state update as fp32 MFMA in
-// the sequential pass. Error against float64, relative norm: outputs 8.4e-7 and
-// state 1.8e-6, as with fp32 products (8.6e-7, 1.6e-6): it is that of exp(G).
+// registers, a few at a time between the chunk's products: 172 KB per chunk and
+// CU take 1.1 us of the CU's load path at 64 bytes per clock, which issued in one
+// go would come on top of the products' time.
+// 4096 tokens of 32 heads: 275 us (pass 1 142, pass 2 140 of it under the
+// tracer), against 359 for the same chunk algorithm with all of T (b V - b g K
+// S_0), Q S_0 + A D and the state update as fp32 MFMA in the sequential pass, and
+// 223 with two f16 parts per operand. Error against float64, relative norm:
+// outputs 8.4e-7 (fp32 MFMA 8.4e-7), state 1.5e-6 (1.5e-6); 200 tokens of 48
+// heads, state 1.6e-7 (fp32 1.7e-7, two f16 parts 1.8e-7). Two chunks
+// do not gain from pass 1's extra work: 128 tokens 30.4 us, fp32 27.9.
 
 #include <hip/hip_runtime.h>
 
@@ -61,78 +61,85 @@
 #include "lds_barrier.h"
 
 #define GC 64        // max chunk length
-#define GKD 128      // max key_dim of the chunked path
 #define TPAD 65      // LDS row stride of L / T
 #define SPAD 132     // LDS row stride of K / Q rows
 
 typedef float gv4f __attribute__((ext_vector_type(4)));
-typedef _Float16 gh2 __attribute__((ext_vector_type(2)));
-typedef _Float16 gh8 __attribute__((ext_vector_type(8)));
+typedef __bf16 gb2 __attribute__((ext_vector_type(2)));
+typedef __bf16 gb8 __attribute__((ext_vector_type(8)));
 
 // Scratch of one (head, chunk), byte offsets. A fragment is one MFMA operand
-// of 16 rows x 32 contraction elements, [lane][8 halves]: lane (m = lane % 16,
-// g = lane / 16) holds row m's elements 4 g .. 4 g + 3 and 16 + 4 g .. + 3 of
+// of 16 rows x 32 contraction elements, [part 3][lane][8 bf16]: lane (m = lane %
+// 16, g = lane / 16) holds row m's elements 4 g .. 4 g + 3 and 16 + 4 g .. + 3 of
 // the 32 (the order in which two 16 x 16 results hold them).
-#define GF_W 0                  // [token strip 4][key step 4][hi, lo][64 lanes][16 B]
-#define GF_K 32768              // K^T: [key tile 8][token step 2][hi, lo]
-#define GF_Q 65536              // as GF_W
-#define GF_A 98304              // [token strip 4][token step 2][hi, lo]
-#define GF_U 114688             // fp32 [value tile 8][token strip 4][64 lanes][4 rows]
-#define GF_AUX 147456           // floats: fw[64], fq[64], fa[64], mu[128], gC, fK, wn
-static_assert(GF_AUX + (3 * 64 + 128 + 3) * 4 <= CTOX_GDN_CHUNK_BYTES, "chunk scratch");
+#define GF_W 0                  // [token strip 4][key step 4] fragments of 3 KB
+#define GF_K 49152              // K^T: [key tile 8][token step 2]
+#define GF_Q 98304              // as GF_W
+#define GF_A 147456             // [token strip 4][token step 2]
+#define GF_U 172032             // fp32 [value tile 8][token strip 4][64 lanes][4 rows]
+#define GF_AUX 204800           // floats: fq[64], gC
+static_assert(GF_AUX + 65 * 4 <= CTOX_GDN_CHUNK_BYTES, "chunk scratch");
 
 __device__ __forceinline__ gv4f mfma4(float a, float b, gv4f c) {
     return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
-__device__ __forceinline__ gv4f mfma_h(uint4 a, uint4 b, gv4f c) {
-    return __builtin_amdgcn_mfma_f32_16x16x32_f16(__builtin_bit_cast(gh8, a), __builtin_bit_cast(gh8, b), c, 0, 0, 0);
+__device__ __forceinline__ gv4f mfma_b(uint4 a, uint4 b, gv4f c) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(gb8, a), __builtin_bit_cast(gb8, b), c, 0, 0, 0);
 }
-// (hi + lo) x (hi + lo) without the lo lo term.
-__device__ __forceinline__ gv4f mfma_split(const uint4 (&a)[2], const uint4 (&b)[2], gv4f c) {
-    c = mfma_h(a[0], b[1], c);
-    c = mfma_h(a[1], b[0], c);
-    return mfma_h(a[0], b[0], c);
-}
+// Product of operands of three parts in three independent chains, the small
+// terms apart from hi hi. Left out: mid lo, lo mid, lo lo, below 2^-23 of hi hi
+// and of either sign.
+struct Acc3 {
+    gv4f c[3] = {};
+    __device__ __forceinline__ void add(const uint4 (&a)[3], const uint4 (&b)[3]) {
+        c[0] = mfma_b(a[2], b[0], c[0]);
+        c[1] = mfma_b(a[1], b[0], c[1]);
+        c[2] = mfma_b(a[0], b[0], c[2]);
+        c[0] = mfma_b(a[1], b[1], c[0]);
+        c[1] = mfma_b(a[0], b[1], c[1]);
+        c[0] = mfma_b(a[0], b[2], c[0]);
+    }
+    __device__ __forceinline__ gv4f sum() const { return (c[0] + c[1]) + c[2]; }
+};
 
-// f16 high and low parts of two values. The values are rounded to fp32 first:
-// a product folded into one use's conversion and not into the other's gives
-// two different high parts next to a rounding boundary.
-__device__ __forceinline__ void split2(float x, float y, uint32_t &hi, uint32_t &lo) {
+// Two values as three bf16 parts each: the high part cut off (no overflow), the
+// rest rounded to the middle one, what is left exactly the low one. The values
+// are rounded to fp32 first: a product folded into one use and not into another
+// gives parts of different values.
+__device__ __forceinline__ void split2(float x, float y, uint32_t &hi, uint32_t &mid, uint32_t &lo) {
     asm("" : "+v"(x), "+v"(y));
-    const gh2 h = {(_Float16)x, (_Float16)y};
-    const gh2 l = {(_Float16)(x - (float)h[0]), (_Float16)(y - (float)h[1])};
-    hi = __builtin_bit_cast(uint32_t, h);
-    lo = __builtin_bit_cast(uint32_t, l);
+    hi = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
+    x -= __uint_as_float(__float_as_uint(x) & 0xffff0000u);
+    y -= __uint_as_float(__float_as_uint(y) & 0xffff0000u);
+    mid = __builtin_bit_cast(uint32_t, (gb2){(__bf16)x, (__bf16)y});
+    x -= __uint_as_float(mid << 16);
+    y -= __uint_as_float(mid & 0xffff0000u);
+    lo = __builtin_amdgcn_perm(__float_as_uint(y), __float_as_uint(x), 0x07060302u);
 }
 // A lane's fragment from two runs of four values.
-__device__ __forceinline__ void split8(gv4f a, gv4f b, uint4 (&f)[2]) {
-    split2(a[0], a[1], f[0].x, f[1].x);
-    split2(a[2], a[3], f[0].y, f[1].y);
-    split2(b[0], b[1], f[0].z, f[1].z);
-    split2(b[2], b[3], f[0].w, f[1].w);
+__device__ __forceinline__ void split8(gv4f a, gv4f b, uint4 (&f)[3]) {
+    split2(a[0], a[1], f[0].x, f[1].x, f[2].x);
+    split2(a[2], a[3], f[0].y, f[1].y, f[2].y);
+    split2(b[0], b[1], f[0].z, f[1].z, f[2].z);
+    split2(b[2], b[3], f[0].w, f[1].w, f[2].w);
 }
-// e with x < 2^e, kept where 2^(15 - e) and 2^(e - 15) are normal numbers
-// (a non-finite x takes the largest).
-__device__ __forceinline__ int exponent_of(float x) {
-    const int e = (int)((__float_as_uint(x) >> 23) & 255u) - 126;
-    return min(128, max(-110, e));
+__device__ __forceinline__ void store3(uint4 *dst, const uint4 (&f)[3]) {
+#pragma unroll
+    for (int x = 0; x < 3; x++) dst[64 * x] = f[x];
 }
-__device__ __forceinline__ float pow2(int e) { return __uint_as_float((uint32_t)(e + 127) << 23); }
+__device__ __forceinline__ void load3(uint4 (&f)[3], const uint4 *src) {
+#pragma unroll
+    for (int x = 0; x < 3; x++) f[x] = src[64 * x];
+}
 
 // exp(x) whose relative error grows with |x| (2^-24 |x|): for decay factors,
 // where |x| exp(x) <= 1/e keeps it under 2^-25 of one.
 __device__ __forceinline__ float exp_decay(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
 
-// Sum / max over the four lane groups (lanes l, l ^ 16, l ^ 32).
+// Sum over the four lane groups (lanes l, l ^ 16, l ^ 32).
 __device__ __forceinline__ float groups_sum(float v) {
     v += __shfl_xor(v, 16);
     return v + __shfl_xor(v, 32);
-}
-__device__ __forceinline__ float groups_max(float v) {
-    auto a = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    v = fmaxf(__uint_as_float((uint32_t)a[0]), __uint_as_float((uint32_t)a[1]));
-    a = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
-    return fmaxf(__uint_as_float((uint32_t)a[0]), __uint_as_float((uint32_t)a[1]));
 }
 
 // 16 x 16 tile of (rows of A) x (rows of B)^T over key_dim on fp32 MFMA: both
@@ -191,7 +198,6 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     __shared__ __align__(16) float kh[GC * SPAD];  // raw K rows, then V rows
     __shared__ float tt[GC * TPAD];                // L, T, W's and then U's left operand
     __shared__ __align__(16) float G[GC], bt[GC], kinv_s[GC], ekf[GC];
-    __shared__ float wmax[4][GC];
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t m16 = lane & 15, g = lane >> 4;
     // A token's heads lie side by side, so the workgroups of one XCD (block % 8)
@@ -228,12 +234,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         const float up = __shfl_up(gl, o);
         if (lane >= (uint32_t)o) gl += up;
     }
-    // The largest exp(G_C - G_r) (1 when no decay exceeds one).
     const float gc = __shfl(gl, 63);
-    float emax = gc - gl;
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) emax = fmaxf(emax, __shfl_xor(emax, o));
-    const int ek = exponent_of(expf(emax));
     if (w == 0) {
         G[lane] = gl;
         bt[lane] = lane < n ? bt_raw : 0.0f;
@@ -255,18 +256,16 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         for (int u = 0; u < 8; u++)
             sq += (qr[u][0] * qr[u][0] + qr[u][1] * qr[u][1]) + (qr[u][2] * qr[u][2] + qr[u][3] * qr[u][3]);
         qinv = own < n ? 1.0f / sqrtf(groups_sum(sq) + 1e-6f) : 0.0f;
-        const float sc = qinv * 16384.0f;
-        uint4 *dst = (uint4 *)(base + GF_Q) + w * 512 + lane;
+        uint4 *dst = (uint4 *)(base + GF_Q) + w * 768 + lane;
 #pragma unroll
         for (int st = 0; st < 4; st++) {
-            uint4 f[2];
-            split8(qr[2 * st] * sc, qr[2 * st + 1] * sc, f);
-            dst[128 * st] = f[0];
-            dst[128 * st + 64] = f[1];
+            uint4 f[3];
+            split8(qr[2 * st] * qinv, qr[2 * st + 1] * qinv, f);
+            store3(dst + 192 * st, f);
         }
     }
     lds_barrier();
-    if (w == 0) ekf[lane] = expf(gc - gl) * kinv_s[lane] * pow2(14 - ek);
+    if (w == 0) ekf[lane] = expf(gc - gl) * kinv_s[lane];
     // 16 x 16 tiles on the raw rows, scaled by the inverse norms afterwards,
     // five per wave: K Q^T of token strip w (rows r, columns t: the result is
     // A's fragment order) and K K^T of strip 3 - w.
@@ -284,7 +283,6 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
             if (u > w) acc[u] = tile_rows(krow + 16 * (u - w - 1) * SPAD, ks);
     }
     {   // A: row t = own, this lane's r = 16 u + 4 g + x
-        float mx = 0.0f;
         const float Gown = G[own];
 #pragma unroll
         for (uint32_t u = 0; u < 4; u++) {
@@ -293,23 +291,16 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 const uint32_t r = 16 * u + 4 * g + x;
-                const float val = r <= own ? exp_decay(Gown - Gr[x]) * (kr4[x] * qinv) * acc[u][x] : 0.0f;
-                acc[u][x] = val;
-                mx = fmaxf(mx, fabsf(val));
+                acc[u][x] = r <= own ? exp_decay(Gown - Gr[x]) * (kr4[x] * qinv) * acc[u][x] : 0.0f;
             }
         }
-        const int e = exponent_of(groups_max(mx));  // (squares of large entries would overflow)
-        const float sc = pow2(14 - e);
-        if (g == 0) aux[128 + own] = qscale * pow2(e - 14);
-        uint4 *dst = (uint4 *)(base + GF_A) + w * 256 + lane;
+        uint4 *dst = (uint4 *)(base + GF_A) + w * 384 + lane;
         const gv4f zero = {0.0f, 0.0f, 0.0f, 0.0f};
-        uint4 f[2];
-        split8(acc[0] * sc, w >= 1 ? acc[1] * sc : zero, f);
-        dst[0] = f[0];
-        dst[64] = f[1];
-        split8(w >= 2 ? acc[2] * sc : zero, w >= 3 ? acc[3] * sc : zero, f);
-        dst[128] = f[0];
-        dst[192] = f[1];
+        uint4 f[3];
+        split8(acc[0], w >= 1 ? acc[1] : zero, f);
+        store3(dst, f);
+        split8(w >= 2 ? acc[2] : zero, w >= 3 ? acc[3] : zero, f);
+        store3(dst + 192, f);
     }
     {   // L of strip 3 - w, strictly lower: the tile's rows are r, its columns s
         const uint32_t s = 16 * (3 - w) + m16;
@@ -345,7 +336,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         for (int s = 0; s < 16; s++) blk[s * TPAD + lane] = col[s];
     }
     {   // K^T fragments of key tiles 2 w, 2 w + 1, with the decay to the chunk's end
-        uint4 *dst = (uint4 *)(base + GF_K) + w * 512 + lane;
+        uint4 *dst = (uint4 *)(base + GF_K) + w * 768 + lane;
 #pragma unroll
         for (int t = 0; t < 2; t++) {
             const float *kp = kh + 16 * (2 * w + t) + m16;
@@ -358,10 +349,9 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
                     lo[x] *= kp[r * SPAD];
                     up[x] *= kp[(r + 16) * SPAD];
                 }
-                uint4 f[2];
+                uint4 f[3];
                 split8(lo, up, f);
-                dst[256 * t + 128 * st] = f[0];
-                dst[256 * t + 128 * st + 64] = f[1];
+                store3(dst + 384 * t + 192 * st, f);
             }
         }
     }
@@ -423,48 +413,27 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
                 wt[st][1] = mfma4(a1, b, wt[st][1]);
             }
         }
-#pragma unroll
-    for (int st = 0; st < 4; st++) {
-        float mx = 0.0f;
-#pragma unroll
-        for (int x = 0; x < 4; x++) mx = fmaxf(mx, fmaxf(fabsf(wt[st][0][x]), fabsf(wt[st][1][x])));
-        mx = groups_max(mx);
-        if (g == 0) wmax[w][16 * st + m16] = mx;
-    }
     lds_barrier();  // K rows and W's left operand are dead
 #pragma unroll
     for (int i = 0; i < 16; i++) tt[(16 * w + i) * TPAD + lane] = tu[i];
 #pragma unroll
     for (int u = 0; u < 8; u++) *(gv4f *)(kh + ((tid >> 5) + 8 * u) * SPAD + (tid & 31) * 4) = vr[u];
     {
-        uint4 *dst = (uint4 *)(base + GF_W) + 128 * w + lane;
+        uint4 *dst = (uint4 *)(base + GF_W) + 192 * w + lane;
 #pragma unroll
         for (int st = 0; st < 4; st++) {
-            const uint32_t s = 16 * st + m16;
-            const int e = exponent_of(fmaxf(fmaxf(wmax[0][s], wmax[1][s]), fmaxf(wmax[2][s], wmax[3][s])));
-            const float sc = pow2(14 - e);
-            uint4 f[2];
-            split8(wt[st][0] * sc, wt[st][1] * sc, f);
-            dst[512 * st] = f[0];
-            dst[512 * st + 64] = f[1];
+            uint4 f[3];
+            split8(wt[st][0], wt[st][1], f);
+            store3(dst + 768 * st, f);
         }
     }
     if (w == 0) {
         const float ge = expf(gl);
-        const float nw = fmaxf(fmaxf(wmax[0][lane], wmax[1][lane]), fmaxf(wmax[2][lane], wmax[3][lane]));
-        aux[lane] = pow2(exponent_of(nw) - 14);
-        aux[64 + lane] = qscale * ge * pow2(-14);
-        float wn = nw;
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) wn = fmaxf(wn, __shfl_xor(wn, o));
-        if (lane == GC - 1) {
-            aux[320] = ge;
-            aux[321] = pow2(ek - 14);
-            aux[322] = wn;
-        }
+        aux[lane] = qscale * ge;
+        if (lane == GC - 1) aux[64] = ge;
     }
     lds_barrier();
-    // U of value tiles 2 w, 2 w + 1 and its largest magnitude per column.
+    // U of value tiles 2 w, 2 w + 1.
     if (32 * w >= dv) return;
     gv4f us[4][2];
 #pragma unroll
@@ -484,64 +453,49 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
         }
     float4 *dst = (float4 *)(base + GF_U) + 512 * w + lane;
 #pragma unroll
-    for (int j = 0; j < 2; j++) {
-        float mx = 0.0f;
+    for (int j = 0; j < 2; j++)
 #pragma unroll
         for (int st = 0; st < 4; st++) {
             const gv4f x = us[st][j];
-            mx = fmaxf(mx, fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3]))));
             dst[256 * j + 64 * st] = make_float4(x[0], x[1], x[2], x[3]);
         }
-        mx = groups_max(mx);
-        if (g == 0) aux[192 + 16 * (2 * w + j) + m16] = mx;
-    }
 }
 
 // A chunk's operands of one wave, in registers one chunk ahead.
 template <int NT>
 struct GdnStateOps {     // waves 0..3
-    uint4 w[4][2];       // W strip, key steps
-    uint4 k[2][2][2];    // K^T key tiles 2 w, 2 w + 1, token steps
-    float4 u[NT], fw;
-    float mu[NT], gc, fk, wn;
+    uint4 w[4][3];       // W strip, key steps
+    uint4 k[2][2][3];    // K^T key tiles 2 w, 2 w + 1, token steps
+    float4 u[NT];
+    float gc;
 };
-template <int NT>
 struct GdnOutOps {       // waves 4..7
-    uint4 q[4][2];
-    uint4 am[2][2];
-    float4 fq, fa;
-    float mu[NT], wn;
+    uint4 q[4][3];
+    uint4 am[2][3];
+    float4 fq;
 };
 
 // The operands' exchange. One buffer each: state operands are read between the
 // first barrier of a chunk and its second, D's after it.
 template <int NT>
 struct GdnScanLds {
-    uint4 s[NT][4][2][64];    // [value tile][key step][hi, lo][lane]
-    uint4 d[NT][2][2][64];    // [value tile][token step][hi, lo][lane]; a strip is half of each 16 B
-    float sf[NT][4][16];      // [value tile][key step][column]: what the state operand was divided by
+    uint4 s[NT][4][3][64];    // [value tile][key step][part][lane]
+    uint4 d[NT][2][3][64];    // [value tile][token step][part][lane]; a strip is half of each 16 B
 };
 
-// X = (rows) x S_0 with the key steps' column factors applied. fetch(k) issues
-// a quarter of the next chunk's loads.
+// X = (rows) x S_0. fetch(k) issues a quarter of the next chunk's loads.
 template <int NT, class Fetch>
-__device__ __forceinline__ gv4f times_state(const uint4 (&x)[4][2], const GdnScanLds<NT> &L, int j, uint32_t lane,
-                                            const float (&sf)[4], Fetch fetch) {
-    gv4f acc[4];
+__device__ __forceinline__ gv4f times_state(const uint4 (&x)[4][3], const GdnScanLds<NT> &L, int j, uint32_t lane,
+                                            Fetch fetch) {
+    Acc3 acc;
 #pragma unroll
     for (int k = 0; k < 4; k++) {
         fetch(k);
         __builtin_amdgcn_sched_barrier(0);
-        const uint4 s[2] = {L.s[j][k][0][lane], L.s[j][k][1][lane]};
-        acc[k] = mfma_split(x[k], s, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+        const uint4 s[3] = {L.s[j][k][0][lane], L.s[j][k][1][lane], L.s[j][k][2][lane]};
+        acc.add(x[k], s);
     }
-    return (acc[0] * sf[0] + acc[1] * sf[1]) + (acc[2] * sf[2] + acc[3] * sf[3]);
-}
-
-// Exponent of D's scale: |D| <= max|U| + max|W| sum|S column|, and a key
-// step's 32 values are below sf 2^15 each.
-__device__ __forceinline__ int d_exponent(float mu, float wn, const float (&sf)[4]) {
-    return exponent_of(mu + wn * (32768.0f * 32.0f) * ((sf[0] + sf[1]) + (sf[2] + sf[3])));
+    return acc.sum();
 }
 
 // NT: value tiles (of 16 columns) per workgroup.
@@ -562,30 +516,17 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
         // part 0..3: W of a key step (and the small operands), 4: K^T of the first key tile, 5: of the second.
         auto load = [&](GdnStateOps<NT> &p, uint32_t c, int part) {
             const char *b = scratch + (size_t)min(c, nch - 1) * CTOX_GDN_CHUNK_BYTES;
-            const uint4 *wp = (const uint4 *)(b + GF_W) + 512 * w + lane, *kp = (const uint4 *)(b + GF_K) + 512 * w + lane;
+            const uint4 *wp = (const uint4 *)(b + GF_W) + 768 * w + lane, *kp = (const uint4 *)(b + GF_K) + 768 * w + lane;
             const float4 *up = (const float4 *)(b + GF_U) + 256 * (NT * slice) + 64 * w + lane;
-            const float *aux = (const float *)(b + GF_AUX);
-            if (part < 4) {
-#pragma unroll
-                for (int x = 0; x < 2; x++) p.w[part][x] = wp[128 * part + 64 * x];
-            }
-            if (part == 0) {
-#pragma unroll
-                for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
-                p.wn = aux[322];
-                p.gc = aux[320];
-                p.fk = aux[321];
-            }
+            if (part < 4) load3(p.w[part], wp + 192 * part);
+            if (part == 0) p.gc = ((const float *)(b + GF_AUX))[64];
             if (part == 1) {
 #pragma unroll
                 for (int j = 0; j < NT; j++) p.u[j] = up[256 * j];
-                p.fw = *(const float4 *)(aux + 16 * w + 4 * g);
             }
             if (part >= 4) {
 #pragma unroll
-                for (int u = 0; u < 2; u++)
-#pragma unroll
-                    for (int x = 0; x < 2; x++) p.k[part - 4][u][x] = kp[256 * (part - 4) + 128 * u + 64 * x];
+                for (int u = 0; u < 2; u++) load3(p.k[part - 4][u], kp + 384 * (part - 4) + 192 * u);
             }
         };
         // State rows 32 w + 16 t + 4 g + r, column j0 + 16 j + m16.
@@ -603,53 +544,39 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
                     st[j][t][r] = i < dk && col < dv ? x : 0.0f;
                 }
         auto publish = [&](int j) {
-            float mx = 0.0f;
-#pragma unroll
-            for (int t = 0; t < 2; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) mx = fmaxf(mx, fabsf(st[j][t][r]));
-            const int e = exponent_of(groups_max(mx));
-            const float sc = pow2(15 - e);
-            uint4 f[2];
-            split8(st[j][0] * sc, st[j][1] * sc, f);
-            L.s[j][w][0][lane] = f[0];
-            L.s[j][w][1][lane] = f[1];
-            if (g == 0) L.sf[j][w][m16] = pow2(e - 15);
+            uint4 f[3];
+            split8(st[j][0], st[j][1], f);
+            store3(&L.s[j][w][0][lane], f);
         };
         auto step = [&](const GdnStateOps<NT> &p, GdnStateOps<NT> &nx, uint32_t c) {
-            float fd[NT];
 #pragma unroll
             for (int j = 0; j < NT; j++) {
-                const float sf[4] = {L.sf[j][0][m16], L.sf[j][1][m16], L.sf[j][2][m16], L.sf[j][3][m16]};
-                const gv4f x = times_state<NT>(p.w, L, j, lane, sf, [&](int k) {
+                const gv4f x = times_state<NT>(p.w, L, j, lane, [&](int k) {
                     if (j == 0) load(nx, c + 1, k);
                 });
-                const int e = d_exponent(p.mu[j], p.wn, sf);
-                const float sc = pow2(15 - e);
-                fd[j] = pow2(e - 15);
-                uint2 hi, lo;
-                split2((p.u[j].x - p.fw.x * x[0]) * sc, (p.u[j].y - p.fw.y * x[1]) * sc, hi.x, lo.x);
-                split2((p.u[j].z - p.fw.z * x[2]) * sc, (p.u[j].w - p.fw.w * x[3]) * sc, hi.y, lo.y);
-                ((uint2 *)&L.d[j][w >> 1][0][lane])[w & 1] = hi;
-                ((uint2 *)&L.d[j][w >> 1][1][lane])[w & 1] = lo;
+                uint2 f[3];
+                split2(p.u[j].x - x[0], p.u[j].y - x[1], f[0].x, f[1].x, f[2].x);
+                split2(p.u[j].z - x[2], p.u[j].w - x[3], f[0].y, f[1].y, f[2].y);
+#pragma unroll
+                for (int i = 0; i < 3; i++) ((uint2 *)&L.d[j][w >> 1][i][lane])[w & 1] = f[i];
             }
             lds_barrier();
 #pragma unroll
             for (int j = 0; j < NT; j++) {
                 if (j == 0) load(nx, c + 1, 4);
-                const uint4 d0[2] = {L.d[j][0][0][lane], L.d[j][0][1][lane]};
-                gv4f n0 = mfma_split(p.k[0][0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
-                gv4f n1 = mfma_split(p.k[1][0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+                Acc3 n0, n1;
+                const uint4 d0[3] = {L.d[j][0][0][lane], L.d[j][0][1][lane], L.d[j][0][2][lane]};
+                n0.add(p.k[0][0], d0);
+                n1.add(p.k[1][0], d0);
                 if (second) {
-                    const uint4 d1[2] = {L.d[j][1][0][lane], L.d[j][1][1][lane]};
-                    n0 = mfma_split(p.k[0][1], d1, n0);
-                    n1 = mfma_split(p.k[1][1], d1, n1);
+                    const uint4 d1[3] = {L.d[j][1][0][lane], L.d[j][1][1][lane], L.d[j][1][2][lane]};
+                    n0.add(p.k[0][1], d1);
+                    n1.add(p.k[1][1], d1);
                 }
                 __builtin_amdgcn_sched_barrier(0);
                 if (j == 0) load(nx, c + 1, 5);
-                const float f = p.fk * fd[j];
-                st[j][0] = st[j][0] * p.gc + n0 * f;
-                st[j][1] = st[j][1] * p.gc + n1 * f;
+                st[j][0] = st[j][0] * p.gc + n0.sum();
+                st[j][1] = st[j][1] * p.gc + n1.sum();
                 publish(j);
             }
             lds_barrier();
@@ -676,40 +603,22 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
                 }
     } else {
         // part 0..3: Q of a key step (and the small operands), 4, 5: A of a token step.
-        auto load = [&](GdnOutOps<NT> &p, uint32_t c, int part) {
+        auto load = [&](GdnOutOps &p, uint32_t c, int part) {
             const char *b = scratch + (size_t)min(c, nch - 1) * CTOX_GDN_CHUNK_BYTES;
-            const uint4 *qp = (const uint4 *)(b + GF_Q) + 512 * w + lane, *ap = (const uint4 *)(b + GF_A) + 256 * w + lane;
-            const float *aux = (const float *)(b + GF_AUX);
-            if (part < 4) {
-#pragma unroll
-                for (int x = 0; x < 2; x++) p.q[part][x] = qp[128 * part + 64 * x];
-            }
-            if (part == 0) {
-#pragma unroll
-                for (int j = 0; j < NT; j++) p.mu[j] = aux[192 + j0 + 16 * j + m16];
-                p.wn = aux[322];
-            }
-            if (part == 1) {
-                p.fq = *(const float4 *)(aux + 64 + 16 * w + 4 * g);
-                p.fa = *(const float4 *)(aux + 128 + 16 * w + 4 * g);
-            }
-            if (part >= 4) {
-#pragma unroll
-                for (int x = 0; x < 2; x++) p.am[part - 4][x] = ap[128 * (part - 4) + 64 * x];
-            }
+            const uint4 *qp = (const uint4 *)(b + GF_Q) + 768 * w + lane, *ap = (const uint4 *)(b + GF_A) + 384 * w + lane;
+            if (part < 4) load3(p.q[part], qp + 192 * part);
+            if (part == 1) p.fq = *(const float4 *)((const float *)(b + GF_AUX) + 16 * w + 4 * g);
+            if (part >= 4) load3(p.am[part - 4], ap + 192 * (part - 4));
         };
         const size_t rowv = (size_t)a.heads * dv;
-        auto step = [&](const GdnOutOps<NT> &p, GdnOutOps<NT> &nx, uint32_t c) {
+        const float qscale = 1.0f / sqrtf((float)dk);
+        auto step = [&](const GdnOutOps &p, GdnOutOps &nx, uint32_t c) {
             gv4f o[NT];
-            float fd[NT];
 #pragma unroll
-            for (int j = 0; j < NT; j++) {
-                const float sf[4] = {L.sf[j][0][m16], L.sf[j][1][m16], L.sf[j][2][m16], L.sf[j][3][m16]};
-                o[j] = times_state<NT>(p.q, L, j, lane, sf, [&](int k) {
+            for (int j = 0; j < NT; j++)
+                o[j] = times_state<NT>(p.q, L, j, lane, [&](int k) {
                     if (j == 0) load(nx, c + 1, k);
                 });
-                fd[j] = pow2(d_exponent(p.mu[j], p.wn, sf) - 15);
-            }
             lds_barrier();
             load(nx, c + 1, 4);
             load(nx, c + 1, 5);
@@ -717,22 +626,24 @@ __device__ __forceinline__ void chunk_scan(const GdnArgs &a) {
             float *out = a.out + (size_t)t0 * rowv + (size_t)h * dv + j0 + m16;
 #pragma unroll
             for (int j = 0; j < NT; j++) {
-                const uint4 d0[2] = {L.d[j][0][0][lane], L.d[j][0][1][lane]};
-                gv4f x = mfma_split(p.am[0], d0, gv4f{0.0f, 0.0f, 0.0f, 0.0f});
+                Acc3 acc;
+                const uint4 d0[3] = {L.d[j][0][0][lane], L.d[j][0][1][lane], L.d[j][0][2][lane]};
+                acc.add(p.am[0], d0);
                 if (w >= 2 && second) {  // strips 0 and 1 see no token of the second step
-                    const uint4 d1[2] = {L.d[j][1][0][lane], L.d[j][1][1][lane]};
-                    x = mfma_split(p.am[1], d1, x);
+                    const uint4 d1[3] = {L.d[j][1][0][lane], L.d[j][1][1][lane], L.d[j][1][2][lane]};
+                    acc.add(p.am[1], d1);
                 }
-                const float fq[4] = {p.fq.x, p.fq.y, p.fq.z, p.fq.w}, fa[4] = {p.fa.x, p.fa.y, p.fa.z, p.fa.w};
+                const gv4f x = acc.sum();
+                const float fq[4] = {p.fq.x, p.fq.y, p.fq.z, p.fq.w};
 #pragma unroll
                 for (int r = 0; r < 4; r++) {
                     const uint32_t s = 16 * w + 4 * g + r;
-                    if (s < n && j0 + 16 * j + m16 < dv) out[(size_t)s * rowv + 16 * j] = fq[r] * o[j][r] + fa[r] * fd[j] * x[r];
+                    if (s < n && j0 + 16 * j + m16 < dv) out[(size_t)s * rowv + 16 * j] = fq[r] * o[j][r] + qscale * x[r];
                 }
             }
             lds_barrier();
         };
-        GdnOutOps<NT> pa, pb;
+        GdnOutOps pa, pb;
 #pragma unroll
         for (int part = 0; part < 6; part++) load(pa, 0, part);
         lds_barrier();

@@ -243,7 +243,7 @@ struct RowDotArgs {
 
 // Chunked prefill: scratch of one (head, chunk), the operands the sequential
 // pass reads (gated_delta_chunk.hip).
-#define CTOX_GDN_CHUNK_BYTES 148992
+#define CTOX_GDN_CHUNK_BYTES 205184
 
 // Gated-delta recurrence. State [heads][key_dim][value_dim] f32.
 struct GdnArgs {

@@ -106,10 +106,9 @@ def test_chunked_prefill_ragged(hip, orc, case):
     (2, 128, 1e6, 1e-3, 1.0, 0.0), (40, 48, 1e-6, 1e5, 1.0, 0.0), (3, 100, 1e30, 1.0, 1.0, 0.0),
     (40, 128, 1e-30, 1e-25, 1.0, 0.0), (2, 16, 1.0, 1.0, 2.0, 0.02), (1, 128, 0.0, 0.0, 1.0, 0.0)])
 def test_chunked_prefill_magnitudes(hip, orc, heads, dv, vs, ss, bmax, ldmax):
-    """The chunked path's operands are split into f16 parts after scaling by
-    powers of two: values and states of any fp32 magnitude (mixed ones too),
-    beta up to 2, decays above one and an all-zero run give what the oracle
-    gives. 40 heads of 48 / 128 columns take the two-tile slices, fewer the
+    """The chunked path's operands are split into 16-bit parts: values and states
+    of any fp32 magnitude, beta up to 2, decays above one and an all-zero run
+    give what the oracle gives. 40 heads of 48 / 128 columns take the two-tile slices, fewer the
     one-tile ones. Tolerances as above, relative to the reference's rms."""
     T, dk, chunk = 200, 128, 64
     say(f"case gdn magnitudes heads={heads} dv={dv} v={vs} s={ss}")
@@ -123,6 +122,35 @@ def test_chunked_prefill_magnitudes(hip, orc, heads, dv, vs, ss, bmax, ldmax):
     got = hip.gated_delta_sequence(q, k, v, ld, be, st_gpu, T, heads, dk, dv, chunk)
     close(got, ref, 1e-3, "output")
     close(st_gpu, st_ref, 1e-4, "state")
+
+
+@pytest.mark.parametrize("heads", [2, 40])
+@pytest.mark.parametrize("what", ["token", "key"])
+def test_chunked_prefill_mixed_magnitudes(hip, orc, heads, what):
+    """Magnitudes 2^40 apart inside one operand, each part judged by its own rms:
+    one late token's values far above the chunk's others (earlier tokens'
+    outputs do not see it), or one key's state row far above the other rows and
+    met by q and k entries as far below theirs. Tolerances as above."""
+    T, dk, dv, big = 64, 128, 64, np.float32(2.0 ** 40)
+    say(f"case gdn mixed magnitudes {what} heads={heads}")
+    q, k, v, ld, be = gdn_inputs(T, heads, heads, dk, dv, 31 + heads)
+    st_ref = np.random.default_rng(heads).standard_normal((heads, dk, dv)).astype(np.float32)
+    if what == "token":
+        v[50] *= big
+    else:
+        st_ref[:, 37] *= big
+        for x in (q, k):
+            x.reshape(T, heads, dk)[:, :, 37] /= big
+    st_ref = st_ref.reshape(-1)
+    st_gpu = st_ref.copy()
+    ref = orc.gated_delta_sequence(q, k, v, ld, be, st_ref, T, heads, dk, dv)
+    got = hip.gated_delta_sequence(q, k, v, ld, be, st_gpu, T, heads, dk, dv, 64)
+    got, ref = np.reshape(got, (T, -1)), np.reshape(ref, (T, -1))
+    for t in range(T):
+        close(got[t], ref[t], 1e-3, f"output {t}")
+    sg, sr = st_gpu.reshape(heads, dk, dv), st_ref.reshape(heads, dk, dv)
+    for i in range(dk):
+        close(sg[:, i], sr[:, i], 1e-4, f"state row {i}")
 
 
 @pytest.mark.parametrize("beta,ld", [(6.0, -3.0), (3.2, -0.01)])
