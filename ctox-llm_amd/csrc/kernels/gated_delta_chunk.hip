@@ -132,10 +132,6 @@ __device__ __forceinline__ void load3(uint4 (&f)[3], const uint4 *src) {
     for (int x = 0; x < 3; x++) f[x] = src[64 * x];
 }
 
-// exp(x) whose relative error grows with |x| (2^-24 |x|): for decay factors,
-// where |x| exp(x) <= 1/e keeps it under 2^-25 of one.
-__device__ __forceinline__ float exp_decay(float x) { return __builtin_amdgcn_exp2f(x * 1.44269504088896341f); }
-
 // Sum over the four lane groups (lanes l, l ^ 16, l ^ 32).
 __device__ __forceinline__ float groups_sum(float v) {
     v += __shfl_xor(v, 16);
@@ -291,7 +287,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 const uint32_t r = 16 * u + 4 * g + x;
-                acc[u][x] = r <= own ? exp_decay(Gown - Gr[x]) * (kr4[x] * qinv) * acc[u][x] : 0.0f;
+                acc[u][x] = r <= own ? expf(Gown - Gr[x]) * (kr4[x] * qinv) * acc[u][x] : 0.0f;
             }
         }
         uint4 *dst = (uint4 *)(base + GF_A) + w * 384 + lane;
@@ -312,7 +308,7 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
 #pragma unroll
             for (int x = 0; x < 4; x++) {
                 const uint32_t r = 16 * (u - w - 1) + 4 * g + x;
-                tt[s * TPAD + r] = r < s ? exp_decay(Gs - Gr[x]) * (f * kr4[x]) * acc[u][x] : 0.0f;
+                tt[s * TPAD + r] = r < s ? expf(Gs - Gr[x]) * (f * kr4[x]) * acc[u][x] : 0.0f;
             }
         }
     }

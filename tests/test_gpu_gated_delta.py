@@ -153,6 +153,29 @@ def test_chunked_prefill_mixed_magnitudes(hip, orc, heads, what):
         close(sg[:, i], sr[:, i], 1e-4, f"state row {i}")
 
 
+def test_chunked_prefill_decay_factor(hip):
+    """Growth by exp(60 .. 80) between two tokens with one key and query axis:
+    o_1 = exp(ld) b_0 v_0 / sqrt(dk) times the norms' 1 / (1 + 1e-6), in float64.
+    A decay factor within one unit in the last place and ten fp32 roundings of
+    the rest: 12 * 2^-24 = 7e-7 (exp2 of a rounded ld * log2 e: up to 2.6e-6)."""
+    T, heads, dk, dv = 3, 32, 128, 16
+    say("case gdn decay factor")
+    rng = np.random.default_rng(2)
+    q = np.zeros((T, heads, dk), np.float32)
+    q[:, :, 3] = 1.0
+    v = rng.standard_normal((T, heads, dv)).astype(np.float32)
+    ld = np.zeros((T, heads), np.float32)
+    ld[1] = rng.uniform(60, 80, heads)
+    be = np.zeros((T, heads), np.float32)
+    be[0] = rng.uniform(0.2, 0.9, heads)
+    st = np.zeros(heads * dk * dv, np.float32)
+    out = np.reshape(hip.gated_delta_sequence(q.reshape(T, -1), q.reshape(T, -1), v.reshape(T, -1), ld, be, st, T, heads,
+                                              dk, dv, 64), (T, heads, dv))
+    want = (np.exp(ld[1].astype(np.float64)) * be[0] / (1 + 1e-6) / math.sqrt(dk))[:, None] * v[0]
+    np.testing.assert_allclose(out[1], want, rtol=7e-7)
+    np.testing.assert_allclose(out[2], want, rtol=7e-7)
+
+
 @pytest.mark.parametrize("beta,ld", [(6.0, -3.0), (3.2, -0.01)])
 def test_chunked_prefill_repeated_key(hip, orc, beta, ld):
     """A repeated key with beta above 2: the undecayed I + L has an inverse of
