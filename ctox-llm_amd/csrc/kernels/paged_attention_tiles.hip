@@ -22,7 +22,7 @@
 //
 //  O^T += V^T P^T: the step's probabilities go through LDS as fp32, and the
 //  wave that owns a value block rounds P x (V scale) to a 23-bit fixed point
-//  (against the block's largest scale in the step) in three int8 limbs: the B
+//  (against the query's largest product of the step) in three int8 limbs: the B
 //  operand, whose k order is the one the scores' C layout leaves, so a lane
 //  packs its own tokens. The A operand is the codes themselves, dims as rows:
 //  ds_read_b64_tr_b4 hands lane l nibble l % 16 of 16 tokens of its choice, a
@@ -37,9 +37,11 @@
 // Bound by VALU issue and a long start: 1900 VALU instructions per wave and step
 // (the f16 kernel takes 750 per 16-token tile, 3000 for the same tokens), but
 // every wave scores four tiles before the first result. 32768 tokens of 24 / 4
-// heads: 5 rows 30.1 us against 39.5, 1 row 19.8 against 21.3 (the combine's 3 us
-// included). Against float64 the output is off by 1.8e-6 of its norm, 2.4e-5
-// with f16 codes and a separate sum of P x scale.
+// heads: 5 rows 31.4 us against 39.5, 1 row 19.8 against 21.3 (the combine's 3 us
+// included). Against float64 the output is off by 1.2e-6 of its norm (2.4e-5 with
+// f16 codes and a separate sum of P x scale; 1.9e-6 and 1 us less with one fixed
+// point per step from the largest V scale, which a token of large values and no
+// probability takes from all others).
 
 typedef int pt_v2i __attribute__((ext_vector_type(2)));
 #define PT_STEP 256   // tokens per step
@@ -220,12 +222,14 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
         PtTiles t;
         pt_tiles(a, desc, at + 4 * wave, t);
         uint2 kr[4][N], vr[4][N];
+        uint32_t piece = lane;
+        if (Q4) asm volatile("" : "+v"(piece));  // (its loop invariant offsets would not fit the registers)
         auto load = [&](uint2 (&r)[4][N], uint32_t first) {  // first: of the token's blocks
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 const bool q4 = Q4 && ((t.q4 >> i) & 1u);
                 pt_load<N, Q4 ? 17 : 9>(a, t.page[i], t.lo[i], t.hi[i], tb + 16 * i, first * (q4 ? 34 : 18),
-                                        q4 ? a.q4_token_bytes : a.q2_token_bytes, q4 ? 17 : 9, lane, r[i]);
+                                        q4 ? a.q4_token_bytes : a.q2_token_bytes, q4 ? 17 : 9, piece, r[i]);
             }
         };
         load(kr, 4 * h);
@@ -243,7 +247,7 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
         auto stage = [&](uint8_t *rows, int i, const uint2 (&r)[N], uint32_t (&c)[8]) {
             uint32_t sc;
             const bool q4 = Q4 && ((t.q4 >> i) & 1u);
-            pt_stage<N, Q4 ? 17 : 9>(rows, q4 ? 34 : 18, lane, r, c, sc);
+            pt_stage<N, Q4 ? 17 : 9>(rows, q4 ? 34 : 18, piece, r, c, sc);
             if (Q4 && !q4) pt_widen(c);
             const uint32_t j = tb + 16 * i + li;
             return pa_half(j >= t.lo[i] && j < t.hi[i] ? sc : 0u);  // absent tokens have a zero scale
@@ -369,17 +373,28 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
             *(float4 *)&L.p[qt][wave][i][lane][0] = p;
         }
         den = den * alpha + sum;
-        // Value block `wave`: its scales times 2^(22 - e), 2^e above the largest (fp16 scales).
-        uint32_t vb = max(max(L.vmax[0][wave], L.vmax[1][wave]), max(L.vmax[2][wave], L.vmax[3][wave]));
-        vb = __builtin_amdgcn_readfirstlane(vb);
-        const int ex = min(max((int)(vb >> 23) - 126, -24), 17);
-        const float back = vb < 0x7f800000u ? ldexpf(1.0f, ex - 22) : __builtin_nanf("");
-        if (qt == 0) {
-            float4 *v = (float4 *)&L.vsc[wave][4 * lane];
-            const float sc = ldexpf(1.0f, 22 - ex);
-            *v = make_float4(v->x * sc, v->y * sc, v->z * sc, v->w * sc);
-        }
+        const uint32_t vb = max(max(L.vmax[0][wave], L.vmax[1][wave]), max(L.vmax[2][wave], L.vmax[3][wave]));
         lds_barrier();
+        // P x (scale of value block `wave`) of the lane's tokens, and the query's fixed point: 2^e above the
+        // largest product, so that a token of large values and little probability takes no bits from the others.
+        float pv[4][16], mx = 0.0f;
+#pragma unroll
+        for (int w = 0; w < 4; w++)
+#pragma unroll
+            for (int i = 0; i < 4; i++) {
+                const float4 p = *(const float4 *)&L.p[qt][w][i][lane][0];
+                const float4 v = *(const float4 *)&L.vsc[wave][64 * w + 16 * i + 4 * lg];
+                const float pp[4] = {p.x, p.y, p.z, p.w}, vv[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+                for (int c = 0; c < 4; c++) pv[w][4 * i + c] = pp[c] * vv[c];
+#pragma unroll
+                for (int c = 0; c < 4; c += 2)
+                    mx = fmaxf(fmaxf(mx, fabsf(pv[w][4 * i + c])), fabsf(pv[w][4 * i + c + 1]));
+            }
+        mx = pa_max_x32(pa_max_x16(mx));
+        const int ex = min(max((int)(__float_as_uint(mx) >> 23) - 126, -100), 17);
+        const float to_x = __uint_as_float((uint32_t)(127 + 22 - ex) << 23);
+        const float back = vb < 0x7f800000u ? __uint_as_float((uint32_t)(127 - 22 + ex) << 23) : __builtin_nanf("");
         // ---- O^T of the block over the step's tokens
         const uint32_t vrow = (16 * (li >> 2) + 4 * lg + (li & 3)) * PT_RS + blk * wave;
         pa_i4 acc[4][3], ones[3];
@@ -389,18 +404,13 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
 #pragma unroll
             for (int d = 0; d < 4; d++) acc[d][k] = pa_i4{0, 0, 0, 0};
         }
+#pragma unroll
         for (int w = 0; w < 4; w++) {
             if (!__builtin_amdgcn_readfirstlane(L.held[w])) continue;
+            // The sum's low mantissa bits are X + 2^22; + 0x408080 makes it X + 0x808080 (low 24 bits).
             uint32_t z[16];
 #pragma unroll
-            for (int i = 0; i < 4; i++) {
-                const float4 p = *(const float4 *)&L.p[qt][w][i][lane][0];
-                const float4 v = *(const float4 *)&L.vsc[wave][64 * w + 16 * i + 4 * lg];
-                const float pp[4] = {p.x, p.y, p.z, p.w}, vv[4] = {v.x, v.y, v.z, v.w};
-                // The sum's low mantissa bits are X + 2^22; + 0x408080 makes it X + 0x808080 (low 24 bits).
-#pragma unroll
-                for (int c = 0; c < 4; c++) z[4 * i + c] = __float_as_uint(fmaf(pp[c], vv[c], 12582912.0f)) + 0x408080u;
-            }
+            for (int x = 0; x < 16; x++) z[x] = __float_as_uint(fmaf(pv[w][x], to_x, 12582912.0f)) + 0x408080u;
             uint32_t l[3][4];
 #pragma unroll
             for (int x = 0; x < 4; x++) {  // tokens in the order the nibbles unpack: even, odd, of 8 each

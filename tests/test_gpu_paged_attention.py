@@ -184,6 +184,33 @@ def test_paged_attention_long(hip, tokens, rows, page, sink, recent, special):
     np.testing.assert_allclose(got[finite], want[finite], rtol=0, atol=8e-5)
 
 
+def test_paged_attention_long_peaked_on_small_value(hip):
+    """The softmax of every query is one token (another step for each KV head)
+    whose values are 1e-3 or less, among tokens with value scales of 1e-3 .. 1e3:
+    every output block is that token's block. Its query score is 64 / 4 c = 16 c
+    above the others' deviation, so their weight is below e^-40 in all; what is
+    left are the 23-bit products and fp32 sums: 2e-5 of the block is ample."""
+    tokens, rows, page, at = 4600, 5, 16, (100, 1500, 3000, 4590)
+    say(f"case paged attention long, peaked on a small value, tokens={tokens} rows={rows}")
+    rng = np.random.default_rng(17)
+    dev, ref = make_caches(hip, tokens + 8, page, 128, 256)
+    k = rng.standard_normal((tokens, KVH, HD)).astype(np.float32)
+    v = rng.standard_normal((tokens, KVH, HD)).astype(np.float32)
+    v *= np.repeat(10.0 ** rng.uniform(-3, 3, (tokens, KVH, HD // 64)), 64, axis=2).astype(np.float32)
+    q = (0.5 * rng.standard_normal((rows, QH, HD))).astype(np.float32)
+    for h in range(KVH):
+        u = rng.standard_normal(HD).astype(np.float32)
+        q[:, h * QH // KVH:(h + 1) * QH // KVH] += 4 * u
+        k[at[h], h] = u
+        v[at[h], h] = 1e-3 * rng.uniform(-1, 1, HD)
+    push_both(dev, ref, k.reshape(tokens, -1), v.reshape(tokens, -1))
+    got = dev.attention(torch.from_numpy(q).cuda(), rows, QH).cpu().numpy().reshape(rows, QH, HD // 64, 64)
+    want = pk.paged_attention(ref, q, rows, QH, KVH, HD).reshape(rows, QH, HD // 64, 64)
+    top = np.abs(want).max(axis=-1, keepdims=True)
+    assert top.max() < 2e-3
+    assert np.all(np.abs(got - want) <= 2e-5 * top), float((np.abs(got - want) / top).max())
+
+
 def test_paged_attention_errors(hip):
     import ctox_hip
     from ctox_hip.paged_kv import DevicePagedKvCache
