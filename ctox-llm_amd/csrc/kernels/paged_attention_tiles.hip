@@ -15,8 +15,8 @@
 //
 //  Scores S = K Q^T, per 64-dim block: a 4 x 4 lane transpose leaves a lane
 //  quarter lg of each of its token's blocks, which is its A operand, as bytes
-//  2 code. The query is a fixed point X of 22 bits per query row, in three
-//  balanced int8 limbs, and sum X (2 code - K) (K = 3 Q2, 15 Q4) is formed in
+//  2 code. The query is a fixed point X of 22 bits per block, in three balanced
+//  int8 limbs, and sum X (2 code - K) (K = 3 Q2, 15 Q4) is formed in
 //  int32 exactly: the -K sum X enters as the MFMA's C operand. One conversion
 //  and one fma with the block's scale per (token, query, block).
 //
@@ -59,7 +59,7 @@ struct PtLds {
     float smax[4][R][16];
     uint32_t vmax[4][4];             // [wave][block]: largest |V scale| (bits)
     uint32_t held[4];                // [wave]: whether it has a token
-    float qs[16 * R];                // score per unit of (block scale x integer sum), base 2
+    float4 qs[16 * R];               // [query], a block each: score per unit of (key scale x integer sum), base 2
     int32_t xs[16 * R][4];           // [query][block]: sum of X
     float den[4][R][16];
 };
@@ -84,7 +84,7 @@ __device__ __forceinline__ uint32_t pt_row_umax(uint32_t v) {
 }
 
 // Queries to limbs: thread i takes (query, block, quarter) = (i / 16, i / 4 % 4,
-// i % 4). X = rint(q 2^E), |X| <= 2^21, E from the query row's largest |q|. A
+// i % 4). X = rint(q 2^E), |X| <= 2^21, E from the query block's largest |q|. A
 // quarter's 16 dims are stored as byte 4 j + i of dim 4 i + j, the order in which
 // a word's four crumbs (or re-paired nibbles) unpack.
 template <int R>
@@ -93,7 +93,8 @@ __device__ __forceinline__ void pt_prep(const GqaArgs &a, const float (&q)[16], 
     float mx = 0.0f;
 #pragma unroll
     for (int d = 0; d < 16; d++) mx = fmaxf(mx, fabsf(q[d]));
-    mx = __uint_as_float(pt_row_umax(__float_as_uint(mx)));  // (magnitudes order as their bits)
+    mx = fmaxf(mx, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(mx), 0xB1, 0xF, 0xF, false)));
+    mx = fmaxf(mx, __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(mx), 0x4E, 0xF, 0xF, false)));
     int ex = 0;
     frexpf(mx, &ex);  // mx < 2^ex
     const float e = mx > 0.0f ? ldexpf(1.0f, 21 - ex) : 0.0f;
@@ -113,8 +114,10 @@ __device__ __forceinline__ void pt_prep(const GqaArgs &a, const float (&q)[16], 
         *(uint4 *)&L.limbs[k][qi][64 * b + 16 * part] = make_uint4(l[k][0], l[k][1], l[k][2], l[k][3]);
     sum += __builtin_amdgcn_update_dpp(0, sum, 0xB1, 0xF, 0xF, false);  // the quad's lanes
     sum += __builtin_amdgcn_update_dpp(0, sum, 0x4E, 0xF, 0xF, false);
-    if (part == 0) L.xs[qi][b] = sum;
-    if (b == 0 && part == 0) L.qs[qi] = mx > 0.0f ? ldexpf(a.scale * PA_LOG2E, ex - 21) : 0.0f;
+    if (part == 0) {
+        L.xs[qi][b] = sum;
+        ((float *)&L.qs[qi])[b] = mx > 0.0f ? ldexpf(a.scale * PA_LOG2E, ex - 21) : 0.0f;
+    }
 }
 
 // Where a wave's four tiles of a step lie (uniform).
@@ -282,6 +285,8 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
             // compiler from holding all of them in registers across steps.
             uint32_t qoff = qi * PA_QB + 16 * lg;
             asm volatile("" : "+v"(qoff));
+            const float4 qs4 = L.qs[qi];
+            const float qs[4] = {qs4.x, qs4.y, qs4.z, qs4.w};
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 if (Q4) {  // quarter q of a block is words 2 q, 2 q + 1
@@ -318,7 +323,7 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
                     const float4 f = *(const float4 *)&L.ksc[wv][i][b][4 * lg];
-                    const float fb[4] = {f.x, f.y, f.z, f.w};
+                    const float fb[4] = {f.x * qs[b], f.y * qs[b], f.z * qs[b], f.w * qs[b]};
                     const pa_i4 a0 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak[i], qv[0], pa_i4{c0, c0, c0, c0}, 0, 0, 0);
                     const pa_i4 a1 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak[i], qv[1], pa_i4{0, 0, 0, 0}, 0, 0, 0);
                     const pa_i4 a2 = __builtin_amdgcn_mfma_i32_16x16x64_i8(ak[i], qv[2], pa_i4{0, 0, 0, 0}, 0, 0, 0);
@@ -332,14 +337,10 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
         }
         float mt = -INFINITY;
         if (any) {
-            const float qs = L.qs[qi];
 #pragma unroll
             for (int i = 0; i < 4; i++)
 #pragma unroll
-                for (int c = 0; c < 4; c++) {
-                    s[i][c] *= qs;
-                    asm volatile("" : "+v"(s[i][c]));  // (formed here, not in the branch below)
-                }
+                for (int c = 0; c < 4; c++) asm volatile("" : "+v"(s[i][c]));  // (formed here, not in the branch below)
             if (!whole) {
 #pragma unroll
                 for (int i = 0; i < 4; i++)

@@ -211,6 +211,27 @@ def test_paged_attention_long_peaked_on_small_value(hip):
     assert np.all(np.abs(got - want) <= 2e-5 * top), float((np.abs(got - want) / top).max())
 
 
+@pytest.mark.parametrize("tokens,rows", [(4600, 5), (300, 5), (4600, 1)])
+def test_paged_attention_query_block_range(hip, tokens, rows):
+    """Queries with one 64-dim block 1e5 times the others, met by keys as far
+    below: every block's part of a score keeps its bits. A block rounded at 2^-22
+    of its largest (4.5 sigma) moves a score by at most scale * sum |k| * 4.5 *
+    2^-22 = 1/16 * 256 * 0.8 * 4.5 * 2^-22 = 1.4e-5 and the output by twice that of
+    sum p |v| < 1 (2.2 fp16 and fp32 roundings of p and v among it): 8e-5."""
+    say(f"case paged attention query blocks tokens={tokens} rows={rows}")
+    rng = np.random.default_rng(tokens + rows)
+    dev, ref = make_caches(hip, tokens + 8, 16, 32, 64)
+    k = rng.standard_normal((tokens, KVH, HD)).astype(np.float32)
+    v = rng.standard_normal((tokens, KVH * HD)).astype(np.float32)
+    q = rng.standard_normal((rows, QH, HD)).astype(np.float32)
+    q[:, :, 64:128] *= np.float32(1e5)
+    k[:, :, 64:128] *= np.float32(1e-5)
+    push_both(dev, ref, k.reshape(tokens, -1), v)
+    got = dev.attention(torch.from_numpy(q).cuda(), rows, QH).cpu().numpy().reshape(rows, QH, HD)
+    want = pk.paged_attention(ref, q, rows, QH, KVH, HD).reshape(rows, QH, HD)
+    np.testing.assert_allclose(got, want, rtol=0, atol=8e-5)
+
+
 def test_paged_attention_errors(hip):
     import ctox_hip
     from ctox_hip.paged_kv import DevicePagedKvCache
