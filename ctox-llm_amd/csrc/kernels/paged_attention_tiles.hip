@@ -1,11 +1,12 @@
-// Split-KV attention over page-aligned tiles (page_tokens a multiple of 16) for
-// contexts that fill the CUs: both products on int8 MFMA 16x16x64 with exact
-// integer sums. Included after paged_attention.hip (page format, the kernels of
-// smaller contexts and other page sizes) and qmatvec_tiled.hip (transpose4).
+// Split-KV attention of 17 to 32 queries per KV head (a verify pass) over
+// page-aligned tiles (page_tokens a multiple of 16) for contexts that fill the
+// CUs: both products on int8 MFMA 16x16x64 with exact integer sums. Included
+// after paged_attention.hip (page format, the kernels of fewer queries, smaller
+// contexts and other page sizes) and qmatvec_tiled.hip (transpose4).
 //
-// A workgroup takes one KV head and a run of 256-token steps; wave w loads and
-// scores tokens 64 w .. 64 w + 63 of a step (four 16-token tiles), and then
-// owns value dims 64 w .. 64 w + 63 for all of the step's tokens.
+// A workgroup takes one KV head and a run of 256-token steps; wave w of a query
+// tile loads and scores tokens 64 w .. 64 w + 63 of a step (four 16-token tiles),
+// and then owns value dims 64 w .. 64 w + 63 for all of the step's tokens.
 //
 //  A token's K (V) head run is four blocks, 72 bytes Q2 or 136 Q4: consecutive
 //  lanes read its consecutive 8 bytes, and an LDS pass hands lane (li, lg) block
@@ -34,34 +35,37 @@
 // kernels do), pays the O conversion per wave and merges four O's in LDS; here
 // one step's 256 tokens are converted once.
 //
-// Bound by VALU issue and a long start: 1900 VALU instructions per wave and step
+// Bound by VALU issue and a long start: 2000 VALU instructions per wave and step
 // (the f16 kernel takes 750 per 16-token tile, 3000 for the same tokens), but
 // every wave scores four tiles before the first result. 32768 tokens of 24 / 4
-// heads: 5 rows 31.4 us against 39.5, 1 row 19.8 against 21.3 (the combine's 3 us
-// included). Against float64 the output is off by 1.2e-6 of its norm (2.4e-5 with
-// f16 codes and a separate sum of P x scale; 1.9e-6 and 1 us less with one fixed
-// point per step from the largest V scale, which a token of large values and no
-// probability takes from all others).
+// heads, 5 rows: 31.3 us against 39.2 (the combine's 3 us included). (With up to
+// 16 queries, 256 threads, it was the faster one only where the steps just fill
+// the CUs, by up to 4%; 1 row: 6500 tokens 16.2 us against the f16 kernel's 13.3,
+// 16384 16.5 / 16.2, 32768 20.7 / 21.3, 32773 32.5 / 24.3, 131072 59.6 / 53.7.)
+// Against float64 the output is off by 1.2e-6 of its norm (2.4e-5 with f16 codes
+// and a separate sum of P x scale; 1.9e-6 and 1 us less with one fixed point per
+// step from the largest V scale, which a token of large values and no probability
+// takes from all others).
 
 typedef int pt_v2i __attribute__((ext_vector_type(2)));
 #define PT_STEP 256   // tokens per step
+#define PT_QT 2       // tiles of 16 queries
 #define PT_RS 136     // LDS bytes of one token's V codes (4 blocks of 32, or 16; + 8: the transposed reads of 64
                       // tokens spread over the banks)
 
-template <int R>
 struct PtLds {
-    int8_t limbs[3][16 * R][PA_QB];
+    int8_t limbs[3][16 * PT_QT][PA_QB];
     uint8_t v[PT_STEP * PT_RS];
-    float p[R][4][4][64][4];         // [query tile][64-token part][token tile][lane][token 4 lg + c]; before
+    float p[PT_QT][4][4][64][4];         // [query tile][64-token part][token tile][lane][token 4 lg + c]; before
                                      // that a wave's part stages its keys
-    float ksc[4 * R][4][4][16];      // [wave][tile][block][token]: K scale / K
+    float ksc[4 * PT_QT][4][4][16];      // [wave][tile][block][token]: K scale / K
     float vsc[4][PT_STEP];           // [block][token]: V scale
-    float smax[4][R][16];
+    float smax[4][PT_QT][16];
     uint32_t vmax[4][4];             // [wave][block]: largest |V scale| (bits)
     uint32_t held[4];                // [wave]: whether it has a token
-    float4 qs[16 * R];               // [query], a block each: score per unit of (key scale x integer sum), base 2
-    int32_t xs[16 * R][4];           // [query][block]: sum of X
-    float den[4][R][16];
+    float4 qs[16 * PT_QT];               // [query], a block each: score per unit of (key scale x integer sum), base 2
+    int32_t xs[16 * PT_QT][4];           // [query][block]: sum of X
+    float den[4][PT_QT][16];
 };
 
 // Bytes of four words, three limbs: l_k holds byte k of z0..z3, as signed digits
@@ -87,8 +91,7 @@ __device__ __forceinline__ uint32_t pt_row_umax(uint32_t v) {
 // i % 4). X = rint(q 2^E), |X| <= 2^21, E from the query block's largest |q|. A
 // quarter's 16 dims are stored as byte 4 j + i of dim 4 i + j, the order in which
 // a word's four crumbs (or re-paired nibbles) unpack.
-template <int R>
-__device__ __forceinline__ void pt_prep(const GqaArgs &a, const float (&q)[16], PtLds<R> &L) {
+__device__ __forceinline__ void pt_prep(const GqaArgs &a, const float (&q)[16], PtLds &L) {
     const uint32_t i = threadIdx.x, qi = i / 16, b = (i / 4) % 4, part = i % 4;
     float mx = 0.0f;
 #pragma unroll
@@ -200,12 +203,11 @@ __device__ __forceinline__ uint4 pt_descs(const GqaArgs &a, uint32_t tile, uint3
     return d;
 }
 
-// grid (splits, kv heads), 256 R threads, R = 1 or 2 tiles of 16 queries: waves 4 qt .. 4 qt + 3 serve
-// query tile qt (both quads read the keys, the first one's V codes are staged for both). A workgroup
-// takes tiles_per_wave tiles (a multiple of 16) from split * tiles_per_wave on.
+// grid (splits, kv heads), 512 threads: waves 4 qt .. 4 qt + 3 serve query tile qt (both quads read the
+// keys, the first one's V codes are staged for both). A workgroup takes tiles_per_wave tiles (a multiple of 16) from split * tiles_per_wave on.
 // Q4: whether a tile of the workgroup lies in a Q4 page (tiles of Q2 pages are then widened).
-template <int R, bool Q4>
-__device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T0, uint32_t T1, uint4 desc) {
+template <bool Q4>
+__device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds &L, uint32_t T0, uint32_t T1, uint4 desc) {
     const uint32_t lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const uint32_t li = lane & 15, lg = lane >> 4, h = blockIdx.y, wave = wv & 3, qt = wv >> 2;
     constexpr float inv_k = Q4 ? 1.0f / 15.0f : 1.0f / 3.0f;
@@ -493,9 +495,8 @@ __device__ __forceinline__ void pt_run(const GqaArgs &a, PtLds<R> &L, uint32_t T
     }
 }
 
-template <int R>
-__device__ __forceinline__ void paged_gqa_tiles(const GqaArgs &a) {
-    __shared__ __align__(16) PtLds<R> L;
+extern "C" __global__ __launch_bounds__(256 * PT_QT, 1) void ctox_paged_gqa_tiles_gfx950(GqaArgs a) {
+    __shared__ __align__(16) PtLds L;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t T0 = blockIdx.x * a.tiles_per_wave, T1 = min(T0 + a.tiles_per_wave, a.tiles);
     const uint4 desc = pt_descs(a, T0, T1, lane);
@@ -503,11 +504,8 @@ __device__ __forceinline__ void paged_gqa_tiles(const GqaArgs &a) {
     pa_prep_load<1>(a, blockIdx.y, qv);
     bool q4 = desc.x != 0;
     for (uint32_t T = T0 + 64; T < T1; T += 64) q4 = q4 || pt_descs(a, T, T1, lane).x != 0;
-    pt_prep<R>(a, qv[0], L);
+    pt_prep(a, qv[0], L);
     lds_barrier();
-    if (__builtin_amdgcn_ballot_w64(q4) == 0) pt_run<R, false>(a, L, T0, T1, desc);
-    else pt_run<R, true>(a, L, T0, T1, desc);
+    if (__builtin_amdgcn_ballot_w64(q4) == 0) pt_run<false>(a, L, T0, T1, desc);
+    else pt_run<true>(a, L, T0, T1, desc);
 }
-
-extern "C" __global__ __launch_bounds__(256, 2) void ctox_paged_gqa_tiles_r1_gfx950(GqaArgs a) { paged_gqa_tiles<1>(a); }
-extern "C" __global__ __launch_bounds__(512, 1) void ctox_paged_gqa_tiles_r2_gfx950(GqaArgs a) { paged_gqa_tiles<2>(a); }

@@ -148,7 +148,7 @@ struct ctox_hip_backend {
                   gdn_scan = nullptr, gdn_chunk_prep[2] = {}, gdn_chunk_scan[2] = {}, gates = nullptr,
                   repeat = nullptr, partials = nullptr, argmax_final = nullptr, greedy_status = nullptr, verify = nullptr, decide = nullptr,
                   pick_sums = nullptr, pick_final = nullptr, rms = nullptr, swiglu = nullptr, sgate = nullptr,
-                  conv = nullptr, rope = nullptr, kv_pack = nullptr, attn_prep = nullptr, kv_demote = nullptr, gqa_part[2] = {}, gqa_part16[2] = {}, gqa_tiles[2] = {},
+                  conv = nullptr, rope = nullptr, kv_pack = nullptr, attn_prep = nullptr, kv_demote = nullptr, gqa_part[2] = {}, gqa_part16[2] = {}, gqa_tiles = nullptr,
                   gqa_combine = nullptr, fill = nullptr, embed = nullptr, norm_rows = nullptr, attn_gate = nullptr,
                   swiglu_rows = nullptr, copy_rows = nullptr, write_words = nullptr, norm_prep = nullptr,
                   prep_x = nullptr, finite = nullptr, gather = nullptr, topk_part = nullptr, topk_final = nullptr, stream_read = nullptr,
@@ -903,8 +903,7 @@ extern "C" ctox_status ctox_hip_backend_create(int device, ctox_hip_backend **ou
                {&b->gqa_part[1], "ctox_paged_gqa_partial_r2_gfx950"},
                {&b->gqa_part16[0], "ctox_paged_gqa_partial16_r1_gfx950"},
                {&b->gqa_part16[1], "ctox_paged_gqa_partial16_r2_gfx950"},
-               {&b->gqa_tiles[0], "ctox_paged_gqa_tiles_r1_gfx950"},
-               {&b->gqa_tiles[1], "ctox_paged_gqa_tiles_r2_gfx950"},
+               {&b->gqa_tiles, "ctox_paged_gqa_tiles_gfx950"},
                {&b->gqa_combine, "ctox_paged_gqa_combine_gfx950"},
                {&b->fill, "ctox_fill_random_gfx950"},      {&b->embed, "ctox_embed_rows_gfx950"},
                {&b->norm_rows, "ctox_norm_rows_gfx950"},   {&b->attn_gate, "ctox_attn_gate_gfx950"},
@@ -2404,18 +2403,12 @@ ctox_status paged_gqa_impl(ctox_hip_backend *b, const float *d_query, const uint
     const uint32_t tiles = (p->tokens + 15) / 16;
     // Two workgroups per CU for the 16-query kernels (they fit two per CU), one for the 32-query ones.
     const bool wide = queries > 16, aligned = p->page_tokens % 16 == 0;
-    const uint32_t per_cu = wide ? 1 : 2, fill = per_cu * (uint32_t)b->cus;
-    // Page-aligned contexts with enough 256-token steps for the CUs take the int8-MFMA kernel; its step
-    // costs less than the f16-MFMA kernel's 16 tiles, its start more, and a CU takes a whole step at a
-    // time. us, int8 against f16, 24 heads over 4 KV heads (4 steps per 256 tokens), 256 CUs:
-    // - More than 16 queries (5 rows): from the length at which an f16 wave gets a second tile; 4096
-    //   tokens (64 steps) 18.8 / 18.7, 6500 18.4 / 20.3, 32768 30.1 / 39.5, 131072 91.5 / 115.
-    // - Up to 16: up to two steps per CU, the last round of CUs seven eighths full; 13000 tokens (204
-    //   steps) 16.2 / 15.5, 16384 15.7 / 16.0 and with 2 rows 16.1 / 17.1, 24000 (376) 20.2 / 19.2, 32768
-    //   (512) 19.8 / 21.3, 131072 (2048) 53.5 / 53.3.
+    const uint32_t fill = (wide ? 1 : 2) * (uint32_t)b->cus;
+    // Page-aligned contexts of more than 16 queries take the int8-MFMA kernel from the length at which an f16
+    // wave gets a second tile. us, int8 against f16, 24 heads over 4 KV heads (4 steps per 256 tokens), 5 rows:
+    // 3000 tokens 18.9 / 17.6, 4100 19.1 / 19.7, 8200 19.8 / 23.9, 32768 31.3 / 39.2, 131072 97.2 / 114.4.
     const uint64_t steps = (uint64_t)((tiles + 15) / 16) * p->key_value_heads;
-    const uint32_t cus = (uint32_t)b->cus, last = (uint32_t)((steps - 1) % cus) + 1;
-    const bool by_step = aligned && (wide ? steps * 4 > fill : steps <= fill && last * 8 > cus * 7);
+    const bool by_step = aligned && wide && steps * 4 > fill;
     const uint32_t unit = by_step ? 16 : 4;  // tiles
     uint32_t splits = std::max<uint32_t>(1, (fill + p->key_value_heads - 1) / p->key_value_heads);
     splits = std::min<uint32_t>(std::min<uint32_t>(splits, (tiles + unit - 1) / unit), 1024);
@@ -2447,8 +2440,8 @@ ctox_status paged_gqa_impl(ctox_hip_backend *b, const float *d_query, const uint
     // Other page-aligned contexts run P.V on f16 MFMA (its waves hold up to 64 tiles' page descriptors in
     // registers), other page sizes the fp32-MFMA kernel.
     const bool f16 = aligned && tpw <= 64;
-    hipFunction_t part_fn = (by_step ? b->gqa_tiles : f16 ? b->gqa_part16 : b->gqa_part)[wide];
-    st = launch(part_fn, dim3(splits, p->key_value_heads), dim3(by_step && wide ? 512 : 256), s, a,
+    hipFunction_t part_fn = by_step ? b->gqa_tiles : (f16 ? b->gqa_part16 : b->gqa_part)[wide];
+    st = launch(part_fn, dim3(splits, p->key_value_heads), dim3(by_step ? 512 : 256), s, a,
                 "ctox_paged_gqa_partial_gfx950");
     if (st) return st;
     return launch(b->gqa_combine, dim3(queries, p->key_value_heads, 4), dim3(256), s, a, "ctox_paged_gqa_combine_gfx950");

@@ -148,9 +148,8 @@ def test_paged_attention_peaked_scores(hip):
     np.testing.assert_allclose(out.cpu().numpy(), want, rtol=1e-3, atol=1e-4 * float(np.abs(want).max()))
 
 
-# Contexts whose 256-token steps fill the CUs (int8 MFMA for both products). 4 KV heads on 256 CUs: from 17
-# steps with more than 16 queries, 57 .. 64 and 121 .. 128 with fewer; 16500 tokens of 5 rows: two steps per
-# workgroup.
+# Long contexts. With more than 16 queries and enough 256-token steps for the CUs both products run on int8 MFMA;
+# 16 queries and fewer stay on f16 MFMA.
 @pytest.mark.parametrize("tokens,rows,page,sink,recent,special", [
     (4353, 5, 16, 16, 16, False),      # the last step holds one token; the first mixes Q4 and Q2 pages
     (4600, 3, 32, 288, 64, True),      # 18 queries; an infinite value scale
