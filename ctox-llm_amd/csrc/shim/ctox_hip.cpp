@@ -2404,17 +2404,27 @@ ctox_status paged_gqa_impl(ctox_hip_backend *b, const float *d_query, const uint
     // Two workgroups per CU for the 16-query kernels (they fit two per CU), one for the 32-query ones.
     const bool wide = queries > 16, aligned = p->page_tokens % 16 == 0;
     const uint32_t fill = (wide ? 1 : 2) * (uint32_t)b->cus;
-    // Page-aligned contexts of more than 16 queries take the int8-MFMA kernel from the length at which an f16
-    // wave gets a second tile. us, int8 against f16, 24 heads over 4 KV heads (4 steps per 256 tokens), 5 rows:
-    // 3000 tokens 18.9 / 17.6, 4100 19.1 / 19.7, 8200 19.8 / 23.9, 32768 31.3 / 39.2, 131072 97.2 / 114.4.
-    const uint64_t steps = (uint64_t)((tiles + 15) / 16) * p->key_value_heads;
-    const bool by_step = aligned && wide && steps * 4 > fill;
-    const uint32_t unit = by_step ? 16 : 4;  // tiles
-    uint32_t splits = std::max<uint32_t>(1, (fill + p->key_value_heads - 1) / p->key_value_heads);
-    splits = std::min<uint32_t>(std::min<uint32_t>(splits, (tiles + unit - 1) / unit), 1024);
-    const uint32_t per_wg = (tiles + unit * splits - 1) / (unit * splits) * unit;
-    splits = (tiles + per_wg - 1) / per_wg;
-    const uint32_t tpw = by_step ? per_wg : per_wg / 4;
+    const uint32_t most = std::max<uint32_t>(1, (fill + p->key_value_heads - 1) / p->key_value_heads);
+    // Splits and tiles per workgroup, a workgroup taking whole units of tiles.
+    auto plan = [&](uint32_t unit, uint32_t &per_wg) {
+        const uint32_t n = std::min<uint32_t>(std::min<uint32_t>(most, (tiles + unit - 1) / unit), 1024);
+        per_wg = (tiles + unit * n - 1) / (unit * n) * unit;
+        return (tiles + per_wg - 1) / per_wg;
+    };
+    uint32_t per_wg, step_wg, splits = plan(4, per_wg);
+    const uint32_t step_splits = plan(16, step_wg);
+    uint32_t tpw = per_wg / 4;
+    // Page-aligned contexts of more than 16 queries take the int8-MFMA kernel where its steps of 256 tokens,
+    // a workgroup taking whole ones, cost less than the f16-MFMA kernel's tiles per wave: 9 + 11 us a step
+    // (step_wg / 16) against 14 + 3.15 us a tile (tpw). us, int8 / f16, 5 rows of 24 heads over 4 KV heads:
+    // 1 step: 3000 tokens (1 tile) 18.9 / 17.6, 4100 (2) 19.1 / 19.7, 16384 (4) 20.4 / 27.0
+    // 2: 16400 (5) 30.7 / 29.9, 20000 (5) 30.4 / 30.2, 22000 (6) 31.2 / 33.1, 32768 (8) 31.3 / 39.2
+    // 3: 32773 (9) 42.4 / 42.6, 40000 (10) 43.2 / 45.9    4: 49200 (13) 53.6 / 54.8    8: 131072 (32) 97 / 114
+    const bool by_step = aligned && wide && 7 * (uint64_t)(step_wg / 16) <= 2 * (uint64_t)tpw + 3;
+    if (by_step) {
+        splits = step_splits;
+        tpw = step_wg;
+    }
     const size_t part = (size_t)p->key_value_heads * splits * queries;
     ctox_status st = ensure(b, b->attn, part * (256 + 2) * sizeof(float), false);
     if (st) return st;
