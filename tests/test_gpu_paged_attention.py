@@ -9,6 +9,7 @@
   rtol 1e-3 plus an absolute 1e-4 x max|out| floor (fp32 MFMA sums in a
   different order than the sequential oracle).
 """
+import math
 import sys
 
 import numpy as np
@@ -229,6 +230,76 @@ def test_paged_attention_query_block_range(hip, tokens, rows):
     got = dev.attention(torch.from_numpy(q).cuda(), rows, QH).cpu().numpy().reshape(rows, QH, HD)
     want = pk.paged_attention(ref, q, rows, QH, KVH, HD).reshape(rows, QH, HD)
     np.testing.assert_allclose(got, want, rtol=0, atol=8e-5)
+
+
+def random_pages(hip, tokens, kvh, page, sink, recent, short, g):
+    """A cache of random packed pages with the retention policy's precisions;
+    short: every 37th page holds a part of its tokens only."""
+    from ctox_hip.paged_kv import DevicePagedKvCache
+    pages, blocks = -(-tokens // page), 2 * kvh * HD // 64
+    first = np.arange(pages) * page
+    count = np.minimum(page, tokens - first)
+    q4 = (first < sink) | (first + count > tokens - recent)
+    if short:
+        count[5:-1:37] = np.maximum(1, count[5:-1:37] * 5 // 8)
+    dev = DevicePagedKvCache(hip, pages * page, kvh, HD, page, sink, recent, q4_slots=int(q4.sum()))
+    for pool, size in ((dev.q4_pool, 34), (dev.q2_pool, 18)):
+        w = torch.randint(0, 256, (pool.numel() // size, size), dtype=torch.uint8, device="cuda", generator=g)
+        w[:, :2] = (0.5 + torch.rand(w.shape[0], device="cuda", generator=g)).half().view(torch.uint8).view(-1, 2)
+        pool.copy_(w.flatten())
+    slot = np.where(q4, np.cumsum(q4), np.cumsum(~q4)) - 1
+    dev.desc[:pages] = np.stack([q4, slot, count, first], 1)
+    dev.d_desc[:pages].copy_(torch.from_numpy(dev.desc[:pages].view(np.int32)))
+    dev.n_pages, dev.n_tokens = pages, tokens
+    return dev
+
+
+def page_values(dev, component, head):
+    """Token values of K (0) or V (1) of a head, float64 [page][token][HD], and the held tokens."""
+    out = torch.zeros(dev.n_pages, dev.page_tokens, HD, dtype=torch.float64, device="cuda")
+    d = torch.from_numpy(dev.desc[:dev.n_pages].astype(np.int64)).cuda()
+    for prec, pool, size, bits in ((1, dev.q4_pool, 34, 4), (0, dev.q2_pool, 18, 2)):
+        pick = d[:, 0] == prec
+        w = pool.view(-1, dev.page_tokens, 2, dev.kv_heads, HD // 64, size)[d[pick, 1]][:, :, component, head]
+        codes = torch.stack([(w[..., 2:] >> b) & (2 ** bits - 1) for b in range(0, 8, bits)], -1).flatten(-2).double()
+        levels = 2 ** bits - 1
+        scale = w[..., :2].contiguous().view(torch.float16).double()
+        out[pick] = (scale * (2 * codes - levels) / levels).flatten(-2)
+    held = torch.arange(dev.page_tokens, device="cuda")[None] < d[:, 2:3]
+    return out.flatten(0, 1), held.flatten()
+
+
+# (KV heads, query heads per KV head, rows, page, tokens, Q4 sink, Q4 recent, short pages)
+@pytest.mark.parametrize("kvh,group,rows,page,tokens,sink,recent,short", [
+    # 8 workgroups of 80 tiles per head: the page descriptors of a workgroup are read twice, the Q4 pages of the
+    # seventh begin past its 64th tile, the last one holds three tiles and a part
+    (32, 1, 17, 16, 9000, 0, 256, False), (32, 1, 17, 16, 9000, 0, 256, True),
+    (4, 6, 5, 16, 22000, 128, 256, True), (4, 6, 5, 128, 40000, 128, 256, True),   # two and three steps of 256
+    (4, 6, 5, 16, 16400, 128, 256, True), (4, 6, 1, 16, 16400, 128, 256, True),    # f16 MFMA
+    (2, 6, 1, 16, 17000, 128, 256, False), (1, 8, 1, 16, 17000, 128, 256, False),  # combines of 133 and 266 splits
+    (1, 8, 4, 16, 17000, 128, 256, False),
+])
+def test_paged_attention_split_paths(hip, kvh, group, rows, page, tokens, sink, recent, short):
+    """Split counts, page descriptors and part-filled pages against a float64
+    softmax over the dequantized pages. Values are below 1.5, 0.58 in the mean
+    square: a query rounded at 2^-22 of its block's largest (4.5 sigma) moves a
+    score by at most 1/16 * 256 * 0.5 * 4.5 * 2^-22 = 9e-6 and the output by twice
+    that of sum p |v| < 1; twice that again for the f16 halves of p: 4e-5."""
+    say(f"case paged attention paths kvh={kvh} group={group} rows={rows} page={page} tokens={tokens} short={short}")
+    g = torch.Generator(device="cuda")
+    g.manual_seed(tokens + rows)
+    dev = random_pages(hip, tokens, kvh, page, sink, recent, short, g)
+    q = torch.randn(rows, kvh * group, HD, device="cuda", generator=g)
+    got = dev.attention(q, rows, kvh * group).view(rows, kvh, group, HD).double()
+    at = torch.arange(dev.n_pages * page, device="cuda")
+    for h in range(kvh):
+        (k, held), (v, _) = page_values(dev, 0, h), page_values(dev, 1, h)
+        qh = q[:, h * group:(h + 1) * group].double().flatten(0, 1)
+        s = qh @ k.T / math.sqrt(HD)
+        row = torch.arange(rows, device="cuda").repeat_interleave(group)
+        s = s.masked_fill(~held[None] | (at[None] > (tokens - rows + row)[:, None]), -math.inf)
+        want = (torch.softmax(s, 1) @ v).view(rows, group, HD)
+        assert float((got[:, h] - want).abs().max()) <= 4e-5, (h, float((got[:, h] - want).abs().max()))
 
 
 def test_paged_attention_errors(hip):
