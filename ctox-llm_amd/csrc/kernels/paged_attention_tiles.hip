@@ -168,6 +168,7 @@ __device__ __forceinline__ void pt_stage(uint8_t *rows, uint32_t bs, uint32_t la
         const uint32_t e = 64 * n + lane;
         if (e < 16 * P) *(uint2 *)(rows + e / P * PT_RS + 8 * (e % P)) = r[n];
     }
+    lds_wave_order();
     constexpr int W = P == 9 ? 4 : 8;
     const uint32_t start = (lane >> 4) * bs;
     const uint8_t *row = rows + (lane & 15) * PT_RS;
@@ -178,6 +179,7 @@ __device__ __forceinline__ void pt_stage(uint8_t *rows, uint32_t bs, uint32_t la
     for (int i = 0; i <= W; i++) x[i] = w[i];
 #pragma unroll
     for (int i = 0; i < W; i++) codes[i] = __builtin_amdgcn_alignbyte(x[i + 1], x[i], (start + 2) & 3u);
+    lds_wave_order();  // (the caller writes the rows again)
 }
 
 // Q2 codes c as Q4 codes 5 c: (2 * 5 c - 15) / 15 = (2 c - 3) / 3, the same value.

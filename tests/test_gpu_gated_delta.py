@@ -241,16 +241,17 @@ def test_errors(hip):
         hip.gated_delta_step([1.0] * 300, [1.0] * 300, [1.0], [0.0], [0.5], np.zeros(300, np.float32), 1, 300, 1)
 
 
-@pytest.mark.parametrize("tokens,chunk", [(1, 0), (5, 0), (40, 16)])
-def test_strided_repeated_key_heads(hip, orc, tokens, chunk):
+# 550 tokens of chunk 16: three runs of chunks share the scratch; a padding of 97 leaves the rows unaligned.
+@pytest.mark.parametrize("tokens,chunk,pad", [(1, 0, 96), (5, 0, 96), (40, 16, 96), (550, 16, 96), (550, 16, 97)])
+def test_strided_repeated_key_heads(hip, orc, tokens, chunk, pad):
     """q, k, v read in place from a fused [q | k | v] token row with 16 key
     heads repeated to 48 value heads (Q/src/decoder.rs:868-913) against the
     oracle on explicitly repeated inputs."""
     import torch
-    print(f"case gdn strided tokens={tokens} chunk={chunk}", flush=True)
+    print(f"case gdn strided tokens={tokens} chunk={chunk} pad={pad}", flush=True)
     rng = np.random.default_rng(tokens + chunk)
     hk, hv, d = 16, 48, 128
-    width = 2 * hk * d + hv * d + 96          # padded token row
+    width = 2 * hk * d + hv * d + pad         # padded token row
     row = (rng.standard_normal((tokens, width))).astype(np.float32)
     q = row[:, :hk * d].reshape(tokens, hk, d)
     k = row[:, hk * d:2 * hk * d].reshape(tokens, hk, d)
