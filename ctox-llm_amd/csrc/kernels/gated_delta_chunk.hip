@@ -52,8 +52,9 @@
 // S_0), Q S_0 + A D and the state update as fp32 MFMA in the sequential pass, and
 // 223 with two f16 parts per operand. Error against float64, relative norm:
 // outputs 8.4e-7 (fp32 MFMA 8.4e-7), state 1.5e-6 (1.5e-6); 200 tokens of 48
-// heads, state 1.6e-7 (fp32 1.7e-7, two f16 parts 1.8e-7). Two chunks
-// do not gain from pass 1's extra work: 128 tokens 30.4 us, fp32 27.9.
+// heads, state 1.6e-7 (fp32 1.7e-7, two f16 parts 1.8e-7). One and
+// two chunks gain little from pass 1's extra work: 64 tokens 23.7 us, 128 tokens
+// 26.4, with fp32 22.9 and 27.9.
 
 #include <hip/hip_runtime.h>
 
@@ -183,12 +184,11 @@ __device__ __forceinline__ gv4f load4(const float *row, uint32_t col, uint32_t w
 }
 
 // Bound by issue and latency: one workgroup is a chain of about a dozen LDS
-// exchanges around 320 fp32 MFMAs per wave (18 us alone on a CU, 13 us of the
-// CU's time each when three share it; without its stores 10% less, without W's
-// and U's products no less). K, Q and V are requested up front, Q stays in
-// registers and V waits in them for K's LDS rows, T replaces L in place, so
-// 52 KB of LDS let three workgroups share a CU (two with Q and T in LDS: 63
-// against 43 us for the 640 workgroups of 20 chunks of 32 heads).
+// exchanges around 320 fp32 MFMAs per wave (17.5 us alone on a CU, 13 us of the
+// CU's time each when three share it; of 33000 clocks the loads take 8500, the
+// tiles with A and L 10500, the inverse 9000, W and U 6000). K, Q and V are
+// requested up front, Q stays in registers and V waits in them for K's LDS rows,
+// T replaces L in place, so 52 KB of LDS let three workgroups share a CU.
 template <bool VEC>
 __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     __shared__ __align__(16) float kh[GC * SPAD];  // raw K rows, then V rows
@@ -196,10 +196,13 @@ __device__ __forceinline__ void chunk_prep(const GdnArgs &a) {
     __shared__ __align__(16) float G[GC], bt[GC], kinv_s[GC], ekf[GC];
     const uint32_t tid = threadIdx.x, lane = tid & 63, w = __builtin_amdgcn_readfirstlane(tid >> 6);
     const uint32_t m16 = lane & 15, g = lane >> 4;
-    // A token's heads lie side by side, so the workgroups of one XCD (block % 8)
-    // take every head: with one XCD's heads 8 apart, their rows fall on the
-    // same few of its L2's channels.
-    const uint32_t h = blockIdx.x / a.chunks, ci = blockIdx.x % a.chunks;
+    // On the XCD that reads the operands in pass 2: lines written on another one
+    // cost both passes (us, this against heads in block order: 128 tokens of 32
+    // heads 26.4 / 30.9, of 48 30.6 / 35.9, 320 of 32 34.3 / 35.4; 1280 and more
+    // within 1%).
+    uint32_t h, ci;
+    head_of_block(blockIdx.x, a.chunks, h, ci);
+    if (h >= a.heads) return;
     const uint32_t t0 = (a.chunk0 + ci) * a.chunk;
     const uint32_t n = min(a.chunk, a.tokens - t0);
     const uint32_t dk = a.key_dim, dv = a.value_dim;

@@ -1774,7 +1774,7 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
         // 16-byte reads of the q, k and v rows.
         const int vec = kd % 4 == 0 && vd % 4 == 0 && qk_stride % 4 == 0 && v_stride % 4 == 0 &&
                         (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
-        const unsigned heads8 = (unsigned)(8 * ((heads + 7) / 8));  // the kernels' XCD map; surplus workgroups exit
+        const unsigned heads8 = (unsigned)(8 * ((heads + 7) / 8));  // both kernels' XCD map; surplus workgroups exit
         // 16-column slices while every (head, slice) has a CU of its own, else 32, whose products share the
         // loaded operands. 1280 tokens, us, 16 / 32 columns: 32 heads 82 / 96, 40 heads 137 / 117, 48 heads
         // 148 / 125, 64 heads 169 / 152.
@@ -1782,7 +1782,7 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
         for (size_t c0 = 0; c0 < nch; c0 += run) {
             a.chunk0 = (uint32_t)c0;
             a.chunks = (uint32_t)std::min(run, nch - c0);
-            st = launch(b->gdn_chunk_prep[vec], dim3((unsigned)heads * a.chunks), dim3(256), s, a, "ctox_gdn_chunk_prep_gfx950");
+            st = launch(b->gdn_chunk_prep[vec], dim3(heads8 * a.chunks), dim3(256), s, a, "ctox_gdn_chunk_prep_gfx950");
             if (!st)
                 st = launch(b->gdn_chunk_scan[nt - 1], dim3(heads8 * (unsigned)((vd + 16 * nt - 1) / (16 * nt))), dim3(512), s, a,
                             "ctox_gdn_chunk_scan_gfx950");
