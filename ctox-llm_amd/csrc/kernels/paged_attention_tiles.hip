@@ -42,10 +42,9 @@
 // 16 queries, 256 threads, it was the faster one only where the steps just fill
 // the CUs, by up to 4%; 1 row: 6500 tokens 16.2 us against the f16 kernel's 13.3,
 // 16384 16.5 / 16.2, 32768 20.7 / 21.3, 32773 32.5 / 24.3, 131072 59.6 / 53.7.)
-// Against float64 the output is off by 1.2e-6 of its norm (2.4e-5 with f16 codes
-// and a separate sum of P x scale; 1.9e-6 and 1 us less with one fixed point per
-// step from the largest V scale, which a token of large values and no probability
-// takes from all others).
+// Against float64 the output is off by 1.2e-6 of its norm (the f16 kernel's by
+// 1.8e-6; 1.9e-6 and 1 us less with one fixed point per step from the largest V
+// scale, which a token of large values and no probability takes from all others).
 
 typedef int pt_v2i __attribute__((ext_vector_type(2)));
 #define PT_STEP 256   // tokens per step
