@@ -47,8 +47,8 @@
 // registers, a few at a time between the chunk's products: 172 KB per chunk and
 // CU take 1.1 us of the CU's load path at 64 bytes per clock, which issued in one
 // go would come on top of the products' time.
-// 4096 tokens of 32 heads: 275 us (pass 1 142, pass 2 140 of it under the
-// tracer), against 359 for the same chunk algorithm with all of T (b V - b g K
+// 4096 tokens of 32 heads: 284 us (under the tracer three launches of 47 us each
+// for pass 1 and for pass 2), against 359 for the same chunk algorithm with all of T (b V - b g K
 // S_0), Q S_0 + A D and the state update as fp32 MFMA in the sequential pass, and
 // 223 with two f16 parts per operand. Error against float64, relative norm:
 // outputs 8.4e-7 (fp32 MFMA 8.4e-7), state 1.5e-6 (1.5e-6); 200 tokens of 48

@@ -457,7 +457,7 @@ __device__ __forceinline__ void pa_tile(const GqaArgs &a, PaLds<R> &L, uint32_t 
 // with E chosen per tile and block from the largest 2 s / K so that B stays
 // in f16's normal range. The products are P (2 s / K) code 4^c whatever E
 // is; the 4^c is removed at the end and the "- s" part is summed per
-// (query, block) on the VALU (corr).
+// (query, block) over the operands as cut off (corr).
 // ---------------------------------------------------------------------------
 typedef _Float16 pa_h2 __attribute__((ext_vector_type(2)));
 typedef _Float16 pa_h4 __attribute__((ext_vector_type(4)));

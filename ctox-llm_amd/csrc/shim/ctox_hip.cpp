@@ -1714,9 +1714,9 @@ extern "C" ctox_status ctox_hip_recovered_row_matvec(ctox_hip_backend *b, const 
 namespace {
 // Scratch of a run of prefill chunks: runs short enough that the sequential
 // pass finds their operands in the 256 MB Infinity Cache, long enough that the
-// launches fill the CUs. us at 110 / 160 / 215 MB and in one run: 4096 tokens of
-// 32 heads (420 MB in all) 273 / 277 / 303 / 356, 3200 of 48 heads 316 / 312 /
-// 312 / 367.
+// launches fill the CUs. us at 45 / 110 / 160 / 215 MB: 4096 tokens of 32 heads
+// (420 MB in all) 340 / 276 / 287 / 339, 3200 of 48 heads (492 MB) 416 / 321 /
+// 315 / 315.
 constexpr size_t kGdnScratch = (size_t)160 << 20;
 
 ctox_status gdn_shape(size_t tokens, size_t heads, size_t kd, size_t vd) {
@@ -1776,8 +1776,8 @@ ctox_status gdn_device(ctox_hip_backend *b, const float *q, const float *k, cons
                         (((uintptr_t)q | (uintptr_t)k | (uintptr_t)v) & 15) == 0;
         const unsigned heads8 = (unsigned)(8 * ((heads + 7) / 8));  // both kernels' XCD map; surplus workgroups exit
         // 16-column slices while every (head, slice) has a CU of its own, else 32, whose products share the
-        // loaded operands. 1280 tokens, us, 16 / 32 columns: 32 heads 82 / 96, 40 heads 137 / 117, 48 heads
-        // 148 / 125, 64 heads 169 / 152.
+        // loaded operands. 1280 tokens, us, 16 / 32 columns: 32 heads 85 / 96, 40 heads 138 / 118, 48 heads
+        // 151 / 127, 64 heads 171 / 153.
         const int nt = heads * slices <= (size_t)b->cus ? 1 : 2;
         for (size_t c0 = 0; c0 < nch; c0 += run) {
             a.chunk0 = (uint32_t)c0;
