@@ -1714,9 +1714,9 @@ extern "C" ctox_status ctox_hip_recovered_row_matvec(ctox_hip_backend *b, const 
 namespace {
 // Scratch of a run of prefill chunks: runs short enough that the sequential
 // pass finds their operands in the 256 MB Infinity Cache, long enough that the
-// launches fill the CUs. us at 45 / 110 / 160 / 215 MB: 4096 tokens of 32 heads
-// (420 MB in all) 340 / 276 / 287 / 339, 3200 of 48 heads (492 MB) 416 / 321 /
-// 315 / 315.
+// launches fill the CUs. Time at 45 / 110 / 215 MB over that at 160: 4096 tokens
+// of 32 heads (420 MB in all) 1.18 / 0.96 / 1.18, 3200 of 48 heads (492 MB) 1.32 /
+// 1.02 / 1.00.
 constexpr size_t kGdnScratch = (size_t)160 << 20;
 
 ctox_status gdn_shape(size_t tokens, size_t heads, size_t kd, size_t vd) {

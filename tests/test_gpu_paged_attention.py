@@ -217,7 +217,7 @@ def test_paged_attention_query_block_range(hip, tokens, rows):
     below: every block's part of a score keeps its bits. A block rounded at 2^-22
     of its largest (4.5 sigma) moves a score by at most scale * sum |k| * 4.5 *
     2^-22 = 1/16 * 256 * 0.8 * 4.5 * 2^-22 = 1.4e-5 and the output by twice that of
-    sum p |v| < 1 (2.2 fp16 and fp32 roundings of p and v among it): 8e-5."""
+    sum p |v| < 1, 3e-5; the roundings of p and of the sums stay below it: 8e-5."""
     say(f"case paged attention query blocks tokens={tokens} rows={rows}")
     rng = np.random.default_rng(tokens + rows)
     dev, ref = make_caches(hip, tokens + 8, 16, 32, 64)
